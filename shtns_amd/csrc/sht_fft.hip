@@ -222,6 +222,19 @@ __device__ __forceinline__ void twiddles(double2 (&w)[P], const double2 *__restr
     });
 }
 
+// Orders LDS accesses between the lanes of one sequence.  A sequence of at most 64 lanes lies
+// in one wave, whose LDS operations complete in order: no block barrier is needed, only that
+// the compiler keeps the order.
+template <int M>
+__device__ __forceinline__ void seq_sync() {
+    if constexpr (WaveGeom<M>::LQ > 64) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 // Passes S.. of the Stockham FFT on the lane's points v[j] = x[l + LQ j].  Pass S (radix P,
 // p = product of the earlier radices) runs butterflies i = l + LQ b, b < R/P, on inputs
 // x[i + r M/P] = v[b + r R/P], multiplies input r by exp(SGN 2 pi i r k/(pP)), k = i mod p,
@@ -258,9 +271,9 @@ __device__ __forceinline__ void wave_passes(double2 (&v)[WaveGeom<M>::R], double
             }
         });
         if constexpr (!last) {
-            __syncthreads();
+            seq_sync<M>();
             sfor<R>([&](auto jc) { v[decltype(jc)::value] = seq[slot_at<LQ>(l, decltype(jc)::value)]; });
-            __syncthreads();
+            seq_sync<M>();
             wave_passes<M, SGN, S + 1>(v, seq, l, roots);
         }
     }
@@ -310,16 +323,16 @@ __device__ __forceinline__ void wave_passes_split(double2 (&v)[WaveGeom<M>::R], 
             };
             double nx[R];
             put(std::integral_constant<int, 0>{});
-            __syncthreads();
+            seq_sync<M>();
             sfor<R>([&](auto jc) { nx[decltype(jc)::value] = seq[slot_at<LQ>(l, decltype(jc)::value)]; });
-            __syncthreads();
+            seq_sync<M>();
             put(std::integral_constant<int, 1>{});
-            __syncthreads();
+            seq_sync<M>();
             sfor<R>([&](auto jc) {
                 constexpr int j = decltype(jc)::value;
                 v[j] = make_double2(nx[j], seq[slot_at<LQ>(l, j)]);
             });
-            __syncthreads();
+            seq_sync<M>();
             wave_passes_split<M, SGN, S + 1>(v, seq, l, roots);
         }
     }
@@ -704,7 +717,7 @@ __global__ __launch_bounds__(NTB) void fft_synth_coops(const double2 *__restrict
         const double2 wB = c_mul(w, B);
         v[j] = make_double2(A.x - wB.y, A.y + wB.x);
     });
-    __syncthreads();
+    seq_sync<M>();
     wave_passes_split<M, 1, 0>(v, seq, l, roots);
     // z_n out: real parts to rows 2n, then imaginary parts to rows 2n+1
     const unsigned off = 8u * (unsigned)((live ? lat0 + tl : 0) * stt + 2 * row * sp);
@@ -776,21 +789,21 @@ __global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB == 256 
         constexpr int j = decltype(jc)::value;
         v[j] = make_double2(vx[j], seq[slot_at<LQ>(l, j)]);
     });
-    __syncthreads();
+    seq_sync<M>();
     wave_passes_split<M, -1, 0>(v, seq, l, roots);
     // X_k = A + conj(w_k) B with A = (Z_k + conj Z_{M-k})/2, B = (Z_k - conj Z_{M-k})/(2i):
     // Z_{M-k} from LDS, real then imaginary parts
     const double2 wl = roots[l];   // loaded here, not before the passes: their register peak
     double zmx[R];
     sfor<R>([&](auto jc) { seq[slot_at<LQ>(l, decltype(jc)::value)] = v[decltype(jc)::value].x; });
-    __syncthreads();
+    seq_sync<M>();
     sfor<R>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         zmx[j] = seq[(j == 0 && l == 0) ? 0 : slot_at<-LQ>(M - l, j)];
     });
-    __syncthreads();
+    seq_sync<M>();
     sfor<R>([&](auto jc) { seq[slot_at<LQ>(l, decltype(jc)::value)] = v[decltype(jc)::value].y; });
-    __syncthreads();
+    seq_sync<M>();
     sfor<R>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
         const int k = l + LQ * j;
@@ -807,7 +820,7 @@ __global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB == 256 
         }
         v[j] = X;
     });
-    __syncthreads();
+    seq_sync<M>();
     // F out with 16-byte stores, latitude fastest: real parts through LDS, then imaginary parts
     double fx[R];
     sfor<R>([&](auto jc) {
