@@ -162,16 +162,18 @@ extern "C" int cushtns_tune(shtns_cfg c, int nfields) {
     c->tune_synth_ncg = b_ncg;
     c->tune_fft_synth = b_fft;
 
-    // analysis: waves per block x field groups per block x FFT kernel (0 = automatic shape)
+    // analysis: waves per block (one and two fields) x field groups per block x FFT kernel
+    // (0 = automatic shape)
     const int ntiles = (c->nlat_2 + 63) / 64;
     std::vector<int> nws{0};
-    for (int d = 1; d <= 12; ++d)
-        if (ntiles % d == 0 && anal_shape_ok(d, ntiles / d)) nws.push_back(d);
+    if (nfields <= 2)
+        for (int d = 1; d <= 12; ++d)
+            if (ntiles % d == 0 && anal_shape_ok(d, ntiles / d)) nws.push_back(d);
     best = 1e30;
     int b_nw = 0, b_ancg = 0, b_afft = 0;
     for (int nw : nws)
         for (int ncg = 1; ncg <= 2; ++ncg) {
-            if (ncg == 2 && (nfields <= 4 || (nw > 0 && ntiles / nw > 3))) continue;
+            if (ncg == 2 && nfields <= 4) continue;
             for (int fk : fft_kinds) {
                 c->tune_anal_nw = nw;
                 c->tune_anal_ncg = ncg;

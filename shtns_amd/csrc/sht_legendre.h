@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <type_traits>
@@ -456,41 +457,33 @@ void synth_tiles_launch(const LegendreArgs &a, int spec_ltop, double2 *F, long f
 // GR > 1 (4x4x4 path, one tile per wave): GR 16-step groups share one barrier pair and one
 // reduction round (16 GR rows of partial tiles), for batches whose MFMA work per group is
 // too small to cover those fixed costs.
-template <int NW, int NLR, int NCG, int PREC, int NF4 = 0, int NG = 1, int GR = 1>
-__global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
+template <int NW, int NLR, int NF4, int GR = 1>
+__global__ __launch_bounds__(64 * NW) void legendre_anal_kernel(
     const double *__restrict__ xk, const double *__restrict__ x2k, const double *__restrict__ stk,
     const double *__restrict__ wqk, const int *__restrict__ step_ofs, const double2 *__restrict__ ab,
     const double4 *__restrict__ pm, const int *__restrict__ i0tab, const double2 *__restrict__ z0tab,
     const double2 *__restrict__ F, long four_dist, double2 *__restrict__ Q, long spec_dist, int lmax_spec,
     int spec_ltop, int mmax, int mres, int nlat, int nlat_2, int ltr, int imlim, int nfields, int vector_mode,
     double mpos_scale, int lat_weight, int cf_lds, int tile_base) {
-    static_assert(NF4 == 0 || (PREC == 0 && NCG == 1 && NF4 <= 3), "4x4x4 path: FP64, one group of <= 3 fields");
-    static_assert(NG == 1 || (NF4 == 0 && NLR == 1), "several field groups per block: one tile per wave");
-    static_assert(GR == 1 || (GR == 2 && NF4 > 0 && NLR == 1 && NG == 1), "two groups per round: 4x4x4 path, one tile");
+    static_assert(NF4 == 1 || NF4 == 2, "one or two fields");
+    static_assert(GR == 1 || (GR == 2 && NLR == 1), "two groups per round: one tile per wave");
     constexpr int RR = 16 * GR;                   // steps per reduction round
-    constexpr int NA = NF4 ? NF4 : NCG;           // operand / accumulator sets
-    constexpr int NCOL = NF4 ? 4 * NF4 : 16 * NCG;
-    constexpr int NT = 64 * NW * NG;              // threads per block
-    __shared__ double ytile[NW * NG][16][65];
+    constexpr int NCOL = 4 * NF4;
+    constexpr int NT = 64 * NW;                   // threads per block
+    __shared__ double ytile[NW][16][65];
     // cf_lds: the order's recurrence coefficients (alpha_i, beta_i), i < nsteps, are copied to
     // LDS once per block (dynamic LDS), so each 16-step group reads them at LDS latency instead
     // of waiting on scalar loads that miss to HBM
     extern __shared__ double2 cfl[];
     // single-buffered: two barriers per block.  Rows padded to NCOL + 2 doubles: a post-mix read
     // (32 lanes = steps 0..15 of two adjacent columns) then falls on 32 distinct bank pairs
-    __shared__ double red[NG][NW][RR][NCOL + 2];
-    __shared__ double carry[NG][2][NCOL];
-    __shared__ int s_ibeg[NW * NG];
+    __shared__ double red[NW][RR][NCOL + 2];
+    __shared__ double carry[2][NCOL];
+    __shared__ int s_ibeg[NW];
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int tw = NG == 1 ? wave : wave % NW, gw = NG == 1 ? 0 : wave / NW;   // tile wave, field group
-    // block -> (order, field groups), field groups fastest: blocks are dispatched in index
-    // order, so all field groups of the heavy low orders start first
-    const int ngr = gridDim.x / (mmax + 1);
-    const int im = blockIdx.x / ngr;
-    const int fblk = (blockIdx.x - im * ngr) * 4 * NCG * NG;   // first field of the block
-    const int fbase = fblk + gw * 4 * NCG;                    // first field of this wave's group
+    const int im = blockIdx.x;   // blocks are dispatched in index order: the heavy low orders start first
 
     const OrderInfo o = order_info(im, lmax_spec, mmax, mres, (im <= imlim) ? ltr : -1, vector_mode);
     const int nsteps = (im <= imlim) ? o.nsteps : 0;
@@ -515,12 +508,11 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
 
     double za[NLR], zb[NLR], x2v[NLR], sdx[NLR], sdy[NLR];
     int i0v[NLR];
-    using C = Contract<PREC>;
-    typename C::b_t Ereg[NLR][NA][16];
+    double Ereg[NLR][NF4][16];
     int my_ibeg = nsteps, my_imax = 0;
 #pragma unroll
     for (int r = 0; r < NLR; ++r) {
-        const int k = (tile_base + tw + NW * r) * 64 + lane;
+        const int k = (tile_base + wave + NW * r) * 64 + lane;
         const bool kv = (k < nlat_2);
         const int kk = kv ? k : 0;
         x2v[r] = x2k[kk];
@@ -540,20 +532,22 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
         // B operand for K-group kg: latitude tile_base + 4*kg + lane/16, column lane%16 of group c
         // (E.re, E.im, O.re, O.im = weighted N+S, N+S, (N-S) x, (N-S) x).  Branch-free, every
         // load issued before the first use: the block's first MFMA waits for these.
-        const int col = NF4 ? (lane & 3) : (lane & 15), comp = col & 3;
+        const int comp = lane & 3;
         const bool keep = nsteps > 0 && !(o.real_only && (comp & 1));
-        const int kl0 = (tile_base + tw + NW * r) * 64 + (lane >> 4);   // latitude of K-group 0
+        // latitude of K-group 0; K-slot k of K-group 2 p + j is latitude 8 p + 2 k + j of the tile,
+        // as in legendre_anal_shared_kernel (both sum in the same order: equal results)
+        const int kl0 = (tile_base + wave + NW * r) * 64 + 2 * (lane >> 4);
         if constexpr (NLR >= 3) {
 #pragma unroll
-            for (int c = 0; c < NA; ++c) {
-                const int f = NF4 ? fbase + c : fbase + 4 * c + (col >> 2);
+            for (int c = 0; c < NF4; ++c) {
+                const int f = c;
                 const bool fv = keep && f < nfields;
                 const double2 *Ff = F + (size_t)(fv ? f : 0) * four_dist + (size_t)im * nlat;
 #pragma unroll
                 for (int kg = 0; kg < 16; ++kg) {
                     // several tiles per wave: one K-group at a time (loads hoisted together
                     // would need more registers than the tiles' operands leave)
-                    const int kl = kl0 + 4 * kg;
+                    const int kl = kl0 + 8 * (kg >> 1) + (kg & 1);
                     double v = 0.0;
                     if (fv && kl < nlat_2) {
                         const double2 fn = Ff[kl], fs = Ff[nlat - 1 - kl];
@@ -561,7 +555,7 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
                         v = (comp == 0 ? fn.x + fs.x : comp == 1 ? fn.y + fs.y
                              : comp == 2 ? (fn.x - fs.x) * xk[kl] : (fn.y - fs.y) * xk[kl]) * w;
                     }
-                    Ereg[r][c][kg] = C::split(v);
+                    Ereg[r][c][kg] = v;
                 }
             }
         } else {
@@ -574,27 +568,27 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
             constexpr int KB = 4;
             const bool neg = comp & 2;
             const double sgn = neg ? -1.0 : 1.0;
-            const double *Fc[NA];
-            bool fvc[NA];
+            const double *Fc[NF4];
+            bool fvc[NF4];
 #pragma unroll
-            for (int c = 0; c < NA; ++c) {
-                const int f = NF4 ? fbase + c : fbase + 4 * c + (col >> 2);
+            for (int c = 0; c < NF4; ++c) {
+                const int f = c;
                 fvc[c] = keep && f < nfields;
                 Fc[c] = reinterpret_cast<const double *>(F + (size_t)(fvc[c] ? f : 0) * four_dist + (size_t)im * nlat) +
                         (comp & 1);
             }
 #pragma unroll
             for (int kb = 0; kb < 16; kb += KB) {
-                double xq[KB], wq[KB], aq[NA][KB], bq[NA][KB];
+                double xq[KB], wq[KB], aq[NF4][KB], bq[NF4][KB];
 #pragma unroll
                 for (int q = 0; q < KB; ++q) {
-                    const int kl = kl0 + 4 * (kb + q);
+                    const int kl = kl0 + 8 * ((kb + q) >> 1) + (q & 1);
                     const int klx = (kl < nlat_2) ? kl : 0;
                     xq[q] = xk[klx];
                     const double wl = wqk[klx];
                     wq[q] = lat_weight ? wl : ((2 * klx + 1 == nlat) ? 0.5 : 1.0);   // odd grid: equator row once
 #pragma unroll
-                    for (int c = 0; c < NA; ++c) {
+                    for (int c = 0; c < NF4; ++c) {
                         const int klc = (fvc[c] && kl < nlat_2) ? kl : 0;
                         aq[c][q] = Fc[c][2 * klc];
                         bq[c][q] = Fc[c][2 * (nlat - 1 - klc)];
@@ -602,15 +596,15 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
                 }
 #pragma unroll
                 for (int q = 0; q < KB; ++q) {
-                    const int kl = kl0 + 4 * (kb + q);
+                    const int kl = kl0 + 8 * ((kb + q) >> 1) + (q & 1);
 #pragma unroll
-                    for (int c = 0; c < NA; ++c) {
+                    for (int c = 0; c < NF4; ++c) {
                         const double s = fma(sgn, bq[c][q], aq[c][q]);
                         double v = (fvc[c] && kl < nlat_2) ? (neg ? s * xq[q] : s) * wq[q] : 0.0;
                         // computed here, not sunk towards the MFMAs (which would keep every
                         // batch's loaded values live across the prologue)
                         asm volatile("" : "+v"(v));
-                        Ereg[r][c][kb + q] = C::split(v);
+                        Ereg[r][c][kb + q] = v;
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -623,7 +617,7 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
     }
     my_imax = __builtin_amdgcn_readfirstlane(my_imax);
     if (lane == 0) s_ibeg[wave] = my_ibeg;
-    if (threadIdx.x < 2 * NCOL * NG) (&carry[0][0][0])[threadIdx.x] = 0.0;
+    if (threadIdx.x < 2 * NCOL) (&carry[0][0])[threadIdx.x] = 0.0;
     if (cf_lds) {
 #pragma unroll
         for (int q = 0; q < NCF; ++q) {
@@ -634,7 +628,7 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
     }
     __syncthreads();
     int ibeg = nsteps;
-    for (int w = 0; w < NW * NG; ++w) ibeg = min(ibeg, s_ibeg[w]);
+    for (int w = 0; w < NW; ++w) ibeg = min(ibeg, s_ibeg[w]);
     ibeg = __builtin_amdgcn_readfirstlane(ibeg) & ~15;   // block-uniform, scalar from here on
 #pragma unroll
     for (int r = 0; r < NLR; ++r) {
@@ -666,7 +660,7 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
 #pragma unroll
             for (int s = 0; s < 16; ++s) {
                 if (ig + s == i0v[r]) { za[r] = sdx[r]; zb[r] = sdy[r]; }
-                C::store_z(&ytile[wave][s][lane], zb[r]);
+                ytile[wave][s][lane] = zb[r];
                 const double zn = fma(fma(cfg[s].x, x2v[r], cfg[s].y), zb[r], za[r]);
                 za[r] = zb[r];
                 zb[r] = zn;
@@ -674,7 +668,7 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
         } else {
 #pragma unroll
             for (int s = 0; s < 16; ++s) {
-                C::store_z(&ytile[wave][s][lane], zb[r]);
+                ytile[wave][s][lane] = zb[r];
                 const double zn = fma(fma(cfg[s].x, x2v[r], cfg[s].y), zb[r], za[r]);
                 za[r] = zb[r];
                 zb[r] = zn;
@@ -703,12 +697,11 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
             pcz[j] = cf4.z;
             pcp[j] = (ii > 0) ? pmm[ii - 1].y : 0.0;
         }
-        using accA_t = std::conditional_t<NF4 == 0, typename C::acc_t, double>;
-        accA_t acc[GR][NA], acc2[GR][NA];   // two chains per column group (even / odd K-groups)
+        double acc[GR][NF4], acc2[GR][NF4];   // two chains per field (halves of the tile)
 #pragma unroll
         for (int q = 0; q < GR; ++q)
 #pragma unroll
-            for (int c = 0; c < NA; ++c) acc[q][c] = acc2[q][c] = accA_t{};
+            for (int c = 0; c < NF4; ++c) acc[q][c] = acc2[q][c] = 0.0;
 #pragma unroll
         for (int q = 0; q < GR; ++q) {
             double2 cf[16];
@@ -716,49 +709,36 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
 #pragma unroll
             for (int r = 0; r < NLR; ++r) {
                 recur_plain(r, i + 16 * q, cf);
-                typename C::a_t a[16];
+                double a[16];
                 __builtin_amdgcn_s_waitcnt(0xc07f);
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int kg = 0; kg < 16; ++kg) a[kg] = C::load_z(&ytile[wave][lane & 15][4 * kg + (lane >> 4)]);
+                for (int kg = 0; kg < 16; ++kg) a[kg] = ytile[wave][lane & 15][8 * (kg >> 1) + 2 * (lane >> 4) + (kg & 1)];
                 __builtin_amdgcn_s_waitcnt(0xc07f);   // all A operands in registers before the tile is rewritten
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
-                for (int kg = 0; kg < 16; kg += 2)
+                for (int kg = 0; kg < 8; ++kg)
 #pragma unroll
-                    for (int c = 0; c < NA; ++c) {
-                        if constexpr (NF4 > 0) {
-                            acc[q][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[kg], Ereg[r][c][kg], acc[q][c], 0, 0, 0);
-                            acc2[q][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[kg + 1], Ereg[r][c][kg + 1], acc2[q][c], 0, 0, 0);
-                        } else {
-                            acc[q][c] = C::mma(a[kg], Ereg[r][c][kg], acc[q][c]);
-                            acc2[q][c] = C::mma(a[kg + 1], Ereg[r][c][kg + 1], acc2[q][c]);
-                        }
+                    for (int c = 0; c < NF4; ++c) {
+                        acc[q][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[kg], Ereg[r][c][kg], acc[q][c], 0, 0, 0);
+                        acc2[q][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[kg + 8], Ereg[r][c][kg + 8], acc2[q][c], 0, 0, 0);
                     }
             }
         }
 #pragma unroll
         for (int q = 0; q < GR; ++q)
 #pragma unroll
-            for (int c = 0; c < NA; ++c) acc[q][c] += acc2[q][c];
+            for (int c = 0; c < NF4; ++c) acc[q][c] += acc2[q][c];
         const int pb = b & 1;
         __syncthreads();   // previous block's post-mix has finished reading red
-        if constexpr (NF4 > 0) {
-            // 4x4x4 D: step 4 ((lane >> 2) & 3) + (lane >> 4), column lane & 3 of field c
+        // 4x4x4 D: step 4 ((lane >> 2) & 3) + (lane >> 4), column lane & 3 of field c
 #pragma unroll
-            for (int q = 0; q < GR; ++q)
+        for (int q = 0; q < GR; ++q)
 #pragma unroll
-                for (int c = 0; c < NA; ++c)
-                    red[gw][tw][16 * q + 4 * ((lane >> 2) & 3) + (lane >> 4)][4 * c + (lane & 3)] = acc[q][c];
-        } else {
-            // D layout (gfx950): acc[c][j] = D[step row 4*j + lane/16][col lane%16]
-#pragma unroll
-            for (int c = 0; c < NCG; ++c)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) red[gw][tw][C::d_row(j, lane)][16 * c + (lane & 15)] = acc[0][c][j];
-        }
+            for (int c = 0; c < NF4; ++c)
+                red[wave][16 * q + 4 * ((lane >> 2) & 3) + (lane >> 4)][4 * c + (lane & 3)] = acc[q][c];
         __syncthreads();
-        // sum over each group's waves + post-mix
+        // sum over the waves + post-mix
 #pragma unroll
         for (int j = 0; j < NE; ++j) {
             const int e = threadIdx.x + j * NT;
@@ -766,34 +746,31 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
             const int row = e & (RR - 1), col = e / RR;
             const int comp = col & 3;
             const int ii = i + row;
+            const int f = col >> 2;
+            double sum = 0.0;
 #pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                const int f = fblk + g * 4 * NCG + (col >> 2);
-                double sum = 0.0;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) sum += red[g][w][row][col];
-                // step row - 1 of this column: lane - 1 (the whole wave is active here; within
-                // a DPP row for 16-row rounds, a wave-wide shift for 32), or the previous
-                // round's last row
-                double sprev = (GR == 1) ? row_shr1(sum) : __shfl_up(sum, 1);
-                if (row == 0) sprev = carry[g][pb ^ 1][col];
-                if (row == RR - 1 && comp < 2) carry[g][pb][col] = sum;
-                if (f >= nfields || ii >= nsteps_out) continue;
-                const int le = o.mfun + 2 * ii;
-                double v = 0.0;
-                if (ii < nsteps) {
-                    if (comp < 2) {
-                        v = pcx[j] * sum + pcp[j] * sprev;
-                    } else {
-                        v = pcz[j] * sum;
-                    }
+            for (int w = 0; w < NW; ++w) sum += red[w][row][col];
+            // step row - 1 of this column: lane - 1 (the whole wave is active here; within
+            // a DPP row for 16-row rounds, a wave-wide shift for 32), or the previous
+            // round's last row
+            double sprev = (GR == 1) ? row_shr1(sum) : __shfl_up(sum, 1);
+            if (row == 0) sprev = carry[pb ^ 1][col];
+            if (row == RR - 1 && comp < 2) carry[pb][col] = sum;
+            if (f >= nfields || ii >= nsteps_out) continue;
+            const int le = o.mfun + 2 * ii;
+            double v = 0.0;
+            if (ii < nsteps) {
+                if (comp < 2) {
+                    v = pcx[j] * sum + pcp[j] * sprev;
+                } else {
+                    v = pcz[j] * sum;
                 }
-                const int ld = (comp < 2) ? le : le + 1;
-                if (ld <= spec_ltop) {
-                    double out = (ld <= ltr) ? v * qscale : 0.0;
-                    if (o.real_only && (comp & 1)) out = 0.0;
-                    reinterpret_cast<double *>(&Qbase[(size_t)f * spec_dist + ld])[comp & 1] = out;
-                }
+            }
+            const int ld = (comp < 2) ? le : le + 1;
+            if (ld <= spec_ltop) {
+                double out = (ld <= ltr) ? v * qscale : 0.0;
+                if (o.real_only && (comp & 1)) out = 0.0;
+                reinterpret_cast<double *>(&Qbase[(size_t)f * spec_dist + ld])[comp & 1] = out;
             }
         }
     }
@@ -801,68 +778,423 @@ __global__ __launch_bounds__(64 * NW * NG) void legendre_anal_kernel(
     for (int ii = threadIdx.x; ii < nsteps_out; ii += NT) {
         if (ii >= ibeg && ii < ibeg + ((nsteps - ibeg + RR - 1) / RR) * RR) continue;
         const int le = o.mfun + 2 * ii;
-        for (int f = fblk; f < min(nfields, fblk + 4 * NCG * NG); ++f) {
+        for (int f = 0; f < nfields; ++f) {
             double2 *Qf = Qbase + (size_t)f * spec_dist;
             if (le <= spec_ltop) Qf[le] = make_double2(0.0, 0.0);
             if (le + 1 <= spec_ltop) Qf[le + 1] = make_double2(0.0, 0.0);
         }
     }
     if (vector_mode && im == 0 && threadIdx.x == 0) {   // degree 0 of the vector m=0 spectra
-        for (int f = fblk; f < min(nfields, fblk + 4 * NCG * NG); ++f) Qbase[(size_t)f * spec_dist] = make_double2(0.0, 0.0);
+        for (int f = 0; f < nfields; ++f) Qbase[(size_t)f * spec_dist] = make_double2(0.0, 0.0);
     }
 }
 
 // static LDS of legendre_anal_kernel, and whether the order's coefficient table (ltr/2 + 2
 // pairs) fits beside it in the 160 KB of a CU
-constexpr size_t anal_static_lds(int NW, int NG, int NCOL, int GR) {
-    return sizeof(double) * NG * (NW * 16 * 65 + NW * 16 * GR * (NCOL + 2) + 2 * NCOL) + sizeof(int) * NW * NG;
+constexpr size_t anal_static_lds(int NW, int NF4, int GR) {
+    return sizeof(double) * (NW * 16 * 65 + NW * 16 * GR * (4 * NF4 + 2) + 8 * NF4) + sizeof(int) * NW;
 }
 inline bool anal_cf_fits(size_t static_lds, int ltr) {
     return static_lds + sizeof(double2) * (size_t)(ltr / 2 + 2) + 1024 <= 160 * 1024;
 }
 
-template <int NW, int NLR, int NCG, int PREC, int NF4 = 0, int NG = 1, int GR = 1>
-void launch_anal_t(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
-                 int spec_ltop, hipStream_t s, int tile_base = 0) {
+template <int NW, int NLR, int NF4, int GR = 1>
+void launch_anal_few(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
+                     int spec_ltop, hipStream_t s, int tile_base = 0) {
     const DeviceTables *t = a.t;
-    dim3 grid((a.mmax + 1) * ((a.nfields + 4 * NCG * NG - 1) / (4 * NCG * NG)));
     // static LDS of the kernel, and the coefficient table if it fits beside it in 160 KB
-    constexpr int NCOL = NF4 ? 4 * NF4 : 16 * NCG;
-    constexpr size_t static_lds = anal_static_lds(NW, NG, NCOL, GR);
+    constexpr size_t static_lds = anal_static_lds(NW, NF4, GR);
     const size_t cf_bytes = sizeof(double2) * (size_t)(a.ltr / 2 + 2);
     const int cf_lds = anal_cf_fits(static_lds, a.ltr) ? 1 : 0;
     const size_t dyn = cf_lds ? cf_bytes : 0;
-    ensure_lds_limit((const void *)legendre_anal_kernel<NW, NLR, NCG, PREC, NF4, NG, GR>, dyn);
-    hipLaunchKernelGGL((legendre_anal_kernel<NW, NLR, NCG, PREC, NF4, NG, GR>), grid, dim3(64 * NW * NG), dyn, s, t->x, t->x2, t->st,
+    ensure_lds_limit((const void *)legendre_anal_kernel<NW, NLR, NF4, GR>, dyn);
+    hipLaunchKernelGGL((legendre_anal_kernel<NW, NLR, NF4, GR>), dim3(a.mmax + 1), dim3(64 * NW), dyn, s, t->x, t->x2, t->st,
                        t->wq, t->step_ofs, t->ab, t->pm, a.vector_mode ? t->i0v : t->i0,
                        a.vector_mode ? t->z0v : t->z0, F, four_dist, Q, spec_dist,
                        spec_ltop == a.lmax + 1 ? a.lmax + 1 : a.lmax, spec_ltop, a.mmax, a.mres, a.nlat, a.nlat_2,
                        a.ltr, a.imlim, a.nfields, a.vector_mode, a.mpos_scale, a.lat_weight, cf_lds, tile_base);
 }
 
+// ---------------------------------------------------------------------------------------
+// Analysis with the recurrence values shared by the block (three or more fields).
+//
+// Block = CT x TT waves for one order and 4 CT fields.  Per group of 16 steps:
+//   1. the owners of the NTB latitude tiles (wave w < NTB, lane = latitude pair) advance their
+//      recurrences and write the values to LDS (the quadrature weights are folded into the
+//      seeds); the previous group's sums are post-mixed;
+//   2. wave (c, t) contracts column tile c (4 fields) over the t-th part of the latitudes, its
+//      E/O data held in registers as MFMA B operands (KGW K-groups of 4 latitudes); the
+//      TT partial 16 x 16 sums go to LDS.
+// A pair of K-groups is one 16-byte LDS read: K-slot k of K-group 2 p + j is latitude
+// 8 p + 2 k + j, rows of PS doubles with PS = 2 mod 16 (no bank conflicts).
+// Tiles whose functions have not started (first step of the tile beyond the group) are
+// skipped: no recurrence, no LDS reads, no MFMAs.
+//
+// The launch covers latitude pairs tile_base * 64 .. pair_end - 1.  accumulate: add to Q instead
+// of storing (the launches after the first where the latitudes do not fit one block).
+// ---------------------------------------------------------------------------------------
+template <int NTB, int CT, int TT, int H>
+struct AnalGeom {
+    static constexpr int NW = CT * TT, NT = 64 * NW;
+    static constexpr int NTH = NTB / H;            // tiles per half
+    static constexpr int KGW = 16 * NTH / TT;      // K-groups per wave and half
+    static constexpr int PS = 64 * NTH + 2;        // doubles per step row of a recurrence buffer
+    static constexpr int NCOL = 16 * CT;
+    static constexpr int TPO = (NTB + NW - 1) / NW;   // tiles per owner
+    static_assert(NTB % H == 0 && 16 * NTH % TT == 0 && KGW % 2 == 0 && NW <= 16, "analysis block shape");
+    static_assert(H == 1 || TPO == H, "halves: each wave owns one tile of each");
+};
+
+// K-groups of the batch of operand loads that starts at K-group kb: two loads each, beside the
+// kb operands already in registers
+constexpr int anal_batch(int kb, int kgw) {
+    int n = kgw > 64 ? (2 * kgw - kb) / 2 & ~3 : (64 - kb) / 2 & ~3;
+    if (n < 4) n = 4;
+    return n < kgw - kb ? n : kgw - kb;
+}
+
+template <int NTB, int CT, int TT, int H, int PREC>
+__global__ __launch_bounds__(64 * CT * TT) void legendre_anal_shared_kernel(
+    const double *__restrict__ xk, const double *__restrict__ x2k, const double *__restrict__ wqk,
+    const int *__restrict__ step_ofs, const double2 *__restrict__ ab, const double4 *__restrict__ pm,
+    const int *__restrict__ i0tab, const double2 *__restrict__ z0tab, const double2 *__restrict__ F, long four_dist,
+    double2 *__restrict__ Q, long spec_dist, int lmax_spec, int spec_ltop, int mmax, int mres, int nlat, int nlat_2,
+    int ltr, int imlim, int nfields, int vector_mode, double mpos_scale, int lat_weight, int tile_base,
+    int pair_end, int accumulate) {
+    using G = AnalGeom<NTB, CT, TT, H>;
+    using C = Contract<PREC>;
+    constexpr int NT = G::NT, NW = G::NW, NTH = G::NTH, KGW = G::KGW, PS = G::PS, NCOL = G::NCOL, TPO = G::TPO;
+    __shared__ __attribute__((aligned(16))) double pt[16 * PS > 128 * NTB ? 16 * PS : 128 * NTB];
+    __shared__ double red[TT][16][NCOL + 2];   // partial sums of the parts
+    __shared__ double carry[2][NCOL];
+    __shared__ double4 pmr[4][16];   // post-mix coefficients of the groups in flight
+    __shared__ int s_tbeg[NTB];
+    __shared__ double2 s_seed[64 * NTB];   // seeds and first steps of the block's latitudes
+    __shared__ int s_i0[64 * NTB];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = wave % CT, t = wave / CT;   // column tile, latitude part
+    const int ngr = gridDim.x / (mmax + 1);
+    const int im = blockIdx.x / ngr;          // field groups fastest: heavy low orders start first
+    const int fbase = (blockIdx.x - im * ngr) * 4 * CT;
+
+    const OrderInfo o = order_info(im, lmax_spec, mmax, mres, (im <= imlim) ? ltr : -1, vector_mode);
+    const int nsteps = (im <= imlim) ? o.nsteps : 0;
+    const int sofs = step_ofs[o.slot];
+    const int last_row = step_ofs[o.slot + 1] - sofs - 1;   // >= nsteps + 6
+    const UniformTable2 abm(ab + sofs);
+
+    // Recurrence state of the owned tiles (every NW-th one; with halves, NTH / NW of each
+    // half).  The seeds wait in LDS: they would cost registers through the whole loop.
+    auto tile_of = [&](int r) { return H == 1 ? wave + NW * r : wave < NTH ? r * NTH + wave : NTB; };
+    int my_ibeg[TPO], my_imax[TPO];
+    double x2[TPO], za[TPO], zb[TPO];
+    double2 sd[TPO];
+#pragma unroll
+    for (int r = 0; r < TPO; ++r) {
+        const int tile = tile_of(r), k = (tile_base + tile) * 64 + lane;
+        const bool kv = tile < NTB && k < pair_end;
+        const int kk = kv ? k : 0;
+        const size_t at = (size_t)o.slot * nlat_2 + kk;
+        x2[r] = x2k[kk];
+        za[r] = zb[r] = 0.0;
+        my_ibeg[r] = kv ? min(i0tab[at], nsteps) : nsteps;
+        sd[r] = z0tab[at];
+    }
+    // cos(theta) and the weights of the block's latitudes, through LDS (the recurrence buffer)
+    constexpr int NX = (64 * NTB + NT - 1) / NT;
+    double *xs = pt, *ws = pt + 64 * NTB;
+    double xv[NX], wv[NX];
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+        const int k = tile_base * 64 + threadIdx.x + q * NT, kx = min(k, nlat_2 - 1);
+        xv[q] = xk[kx];
+        wv[q] = wqk[kx];
+        if (!lat_weight) wv[q] = (2 * kx + 1 == nlat) ? 0.5 : 1.0;   // odd grid: the equator row, both rows of its pair, once
+        if (k >= pair_end) wv[q] = 0.0;
+    }
+    auto put_tables = [&]() {
+#pragma unroll
+        for (int q = 0; q < NX; ++q) {
+            const int e = threadIdx.x + q * NT;
+            if (e < 64 * NTB) { xs[e] = xv[q]; ws[e] = wv[q]; }
+        }
+#pragma unroll
+        for (int r = 0; r < TPO; ++r) {
+            const int tile = tile_of(r);
+            if (tile < NTB) {
+                s_seed[tile * 64 + lane] = sd[r];
+                s_i0[tile * 64 + lane] = my_ibeg[r];
+            }
+        }
+        __syncthreads();
+    };
+
+    // B operands.  The Fourier rows are loaded in as few batches as the registers allow (every
+    // load of a batch in flight before the first is used, the batches fenced): each batch costs
+    // the block a full memory latency.
+    typename C::b_t Breg[H * KGW];
+    {
+        const int col = lane & 15, comp = col & 3, f = fbase + 4 * c + (col >> 2);
+        const bool keep = nsteps > 0 && !(o.real_only && (comp & 1)) && f < nfields;
+        const bool neg = comp & 2;
+        const double sgn = neg ? -1.0 : 1.0;
+        const double *Fc = reinterpret_cast<const double *>(F + (size_t)(keep ? f : 0) * four_dist + (size_t)im * nlat) + (comp & 1);
+        const int kloc = t * KGW * 4 + 2 * (lane >> 4), kl0 = tile_base * 64 + kloc;
+        // latitude offset of K-group n (halves: the part's share of each)
+        auto dk_of = [](int n) { return (n / KGW) * 64 * NTH + 8 * ((n % KGW) >> 1) + (n & 1); };
+        auto load = [&](auto full, auto kbc, auto KBc) {   // K-groups kb .. kb + KB - 1
+            constexpr int kb = decltype(kbc)::value, KB = decltype(KBc)::value;
+            double aq[KB], bq[KB];
+#pragma unroll
+            for (int q = 0; q < KB; ++q) {
+                const int dk = dk_of(kb + q);
+                const int kl = decltype(full)::value ? kl0 + dk : min(kl0 + dk, nlat_2 - 1);
+                aq[q] = Fc[2 * kl];
+                bq[q] = Fc[2 * (nlat - 1 - kl)];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (kb == 0) put_tables();
+#pragma unroll
+            for (int q = 0; q < KB; ++q) {
+                const int e = kloc + dk_of(kb + q);
+                const double s = fma(sgn, bq[q], aq[q]);
+                double v = keep ? (neg ? s * xs[e] : s) * ws[e] : 0.0;
+                asm volatile("" : "+v"(v));
+                Breg[kb + q] = C::split(v);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto all = [&](auto self, auto full, auto kbc) -> void {
+            constexpr int kb = decltype(kbc)::value, n = anal_batch(kb, H * KGW);
+            load(full, kbc, std::integral_constant<int, n>{});
+            if constexpr (kb + n < H * KGW) self(self, full, std::integral_constant<int, kb + n>{});
+        };
+        constexpr std::integral_constant<int, 0> k0{};
+        if ((tile_base + NTB) * 64 <= pair_end) all(all, std::true_type{}, k0);
+        else all(all, std::false_type{}, k0);
+    }
+#pragma unroll
+    for (int r = 0; r < TPO; ++r) {
+        my_imax[r] = my_ibeg[r] < nsteps ? my_ibeg[r] : 0;   // lanes that never start stay zero
+        for (int off = 32; off >= 1; off >>= 1) {
+            my_ibeg[r] = min(my_ibeg[r], __shfl_xor(my_ibeg[r], off));
+            my_imax[r] = max(my_imax[r], __shfl_xor(my_imax[r], off));
+        }
+        my_ibeg[r] = __builtin_amdgcn_readfirstlane(my_ibeg[r]);
+        my_imax[r] = __builtin_amdgcn_readfirstlane(my_imax[r]);
+        if (tile_of(r) < NTB && lane == 0) s_tbeg[tile_of(r)] = my_ibeg[r];
+    }
+    __syncthreads();
+    int ibeg = nsteps;
+    for (int w = 0; w < NTB; ++w) ibeg = min(ibeg, s_tbeg[w]);
+    ibeg = __builtin_amdgcn_readfirstlane(ibeg) & ~15;
+    // first steps of the tiles this wave contracts (one per 16 K-groups, or the one its part is
+    // in; parts that straddle tiles take the first of any of them, and every tile is then written)
+    constexpr bool STRADDLE = !(KGW % 16 == 0 || 16 % KGW == 0);
+    constexpr int TPW = !STRADDLE && KGW >= 16 ? KGW / 16 : 1, KGT = KGW / TPW;
+    int tb[H * TPW];
+#pragma unroll
+    for (int q = 0; q < H * TPW; ++q) {
+        int b = nsteps;
+        const int k0 = t * KGW + (q % TPW) * KGT, h0 = (q / TPW) * NTH;
+        for (int w = k0 / 16; w <= (k0 + KGT - 1) / 16; ++w) b = min(b, s_tbeg[h0 + w]);
+        tb[q] = __builtin_amdgcn_readfirstlane(b);
+    }
+    // the 16 steps from ig of the owned tiles into LDS
+    auto recur = [&](int ig, const double2 *cf, int half) {
+#pragma unroll
+        for (int r = 0; r < TPO; ++r) {
+            if (H > 1 && r != half) continue;
+            if (tile_of(r) >= NTB || (!STRADDLE && ig + 16 <= my_ibeg[r])) continue;   // not started: nobody reads it
+            const int tile = tile_of(r), h = tile / NTH;
+            double *dst = &pt[(tile - h * NTH) * 64 + lane];
+            if (ig <= my_imax[r]) {   // some lane of this wave starts its recurrence here
+                const int i0 = s_i0[tile * 64 + lane];
+                const double2 sd = s_seed[tile * 64 + lane];
+#pragma unroll
+                for (int s = 0; s < 16; ++s) {
+                    if (ig + s == i0) { za[r] = sd.x; zb[r] = sd.y; }
+                    C::store_z(dst + s * PS, zb[r]);
+                    const double zn = fma(fma(cf[s].x, x2[r], cf[s].y), zb[r], za[r]);
+                    za[r] = zb[r];
+                    zb[r] = zn;
+                    if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // few factors ahead: registers
+                }
+            } else {
+#pragma unroll
+                for (int s = 0; s < 16; ++s) {
+                    C::store_z(dst + s * PS, zb[r]);
+                    const double zn = fma(fma(cf[s].x, x2[r], cf[s].y), zb[r], za[r]);
+                    za[r] = zb[r];
+                    zb[r] = zn;
+                    if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // few factors ahead: registers
+                }
+            }
+        }
+    };
+    // coefficients of a group (wave-uniform: scalar loads), clamped to the order's table
+    auto load_cf = [&](double2 *cf, int ig) {
+#pragma unroll
+        for (int s = 0; s < 16; s += 4) {
+            const int i4 = min(ig + s, last_row - 3);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cf[s + q] = abm[i4 + q];
+        }
+    };
+    constexpr bool TWO = PREC == 0 && KGW > 8 && H * KGW < 64;   // two chains (halves of a tile) where registers allow
+    double4_t acc, acc1;
+    const bool active = fbase + 4 * c < nfields;   // the last column tiles of a batch may be empty
+    auto contract = [&](int ig, auto hc) {
+        constexpr int h = decltype(hc)::value;
+        const double *src = &pt[(lane & 15) * PS + t * KGW * 4 + 2 * (lane >> 4)];
+#pragma unroll
+        for (int q = 0; q < TPW; ++q) {
+            if (!active || ig + 16 <= tb[h * TPW + q]) continue;   // wave-uniform
+            constexpr int NQ = KGT / 2;
+            typename C::acc_t part = C::zero();   // FP32 sums over at most 8 K-groups (unused at PREC 0)
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) {
+                // the two chains in turn: pairs 0 .. 3 of a tile to acc, 4 .. 7 to acc1
+                const int p = (TWO && NQ == 8) ? (n >> 1) + 4 * (n & 1) : n;
+                const double2 a2 = *reinterpret_cast<const double2 *>(src + 8 * (q * NQ + p));
+                const typename C::b_t b0 = Breg[h * KGW + q * KGT + 2 * p], b1 = Breg[h * KGW + q * KGT + 2 * p + 1];
+                if constexpr (PREC == 0) {
+                    double4_t &d = (TWO && (p & 4)) ? acc1 : acc;
+                    d = C::mma(a2.x, b0, d);
+                    d = C::mma(a2.y, b1, d);
+                } else {
+                    part = C::mma(C::load_z(&a2.y), b1, C::mma(C::load_z(&a2.x), b0, part));
+                    if (p % 4 == 3 || p == NQ - 1) {
+                        acc += __builtin_convertvector(part, double4_t);
+                        part = C::zero();
+                    }
+                }
+            }
+        }
+    };
+
+    const double qscale = (im == 0) ? 1.0 : mpos_scale;
+    const int nsteps_out = (spec_ltop >= o.mfun) ? (spec_ltop - o.mfun) / 2 + 1 : 0;
+    double2 *Qbase = Q + o.spec_base;
+    // Sum over the parts and post-mix of group i: element e of the 16 x NCOL block is step row
+    // e % 16 of column e / 16, so a 16-lane DPP row holds the 16 steps of one column (the even
+    // degrees' second term takes the neighbouring lane's sum) and a wave stores the 32
+    // consecutive degrees of one field.
+    auto post = [&](int i) {
+        const int slot = (i >> 4) & 3, pb = (i >> 4) & 1;
+        for (int e = threadIdx.x; e < 16 * NCOL; e += NT) {
+            const int row = e & 15, col = e >> 4, comp = col & 3;
+            const int ii = i + row, f = fbase + (col >> 2);
+            double sum = 0.0;
+            if constexpr (TT == 2 * NTB) {   // half-tile parts: tile by tile, as the two chains of whole tiles
+#pragma unroll
+                for (int w = 0; w < TT; w += 2) sum += red[w][row][col] + red[w + 1][row][col];
+            } else {
+#pragma unroll
+                for (int w = 0; w < TT; ++w) sum += red[w][row][col];
+            }
+            double sprev = row_shr1(sum);
+            if (row == 0) sprev = carry[pb ^ 1][col];
+            if (row == 15 && comp < 2) carry[pb][col] = sum;
+            const int ld = o.mfun + 2 * ii + (comp >> 1);
+            if (f >= nfields || ii >= nsteps_out || ld > spec_ltop) continue;
+            double v = 0.0;
+            if (ii < nsteps) {
+                if (comp < 2) v = pmr[slot][row].x * sum + (row ? pmr[slot][row - 1].y : pmr[(slot + 3) & 3][15].y) * sprev;
+                else v = pmr[slot][row].z * sum;
+            }
+            double out = (ld <= ltr) ? v * qscale : 0.0;
+            if (o.real_only && (comp & 1)) out = 0.0;
+            double *q = &reinterpret_cast<double *>(&Qbase[(size_t)f * spec_dist + ld])[comp & 1];
+            *q = accumulate ? *q + out : out;
+        }
+    };
+    auto put_red = [&]() {
+        if constexpr (TWO) acc += acc1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) red[t][C::d_row(j, lane)][16 * c + (lane & 15)] = acc[j];
+    };
+    for (int e = threadIdx.x; e < 2 * NCOL; e += NT) (&carry[0][0])[e] = 0.0;
+    // (the step before the first group's has zero sums: its coefficient only has to be finite)
+    if (threadIdx.x < 4) pmr[threadIdx.x][15] = make_double4(0.0, 0.0, 0.0, 0.0);
+    __syncthreads();
+    int ng = 0;
+    double2 cf[16];
+    load_cf(cf, ibeg);
+    for (int i = ibeg; i < nsteps; i += 16, ++ng) {
+        auto part_of = [&](auto hc) {
+            constexpr int h = decltype(hc)::value;
+            double4 pmv;
+            if (h == 0 && threadIdx.x >= NT - 16) pmv = pm[sofs + min(i + (int)(threadIdx.x & 15), last_row)];
+            recur(i, cf, h);
+            if (h == 0 && ng > 0) post(i - 16);
+            if (h == 0 && threadIdx.x >= NT - 16) pmr[(i >> 4) & 3][threadIdx.x & 15] = pmv;
+            __syncthreads();
+            if (h == H - 1) load_cf(cf, i + 16);   // in flight during the contraction
+            __builtin_amdgcn_sched_barrier(0);
+            if (h == 0) {
+                acc = double4_t{};
+                if constexpr (TWO) acc1 = double4_t{};
+            }
+            contract(i, hc);
+            if (h == H - 1) put_red();
+            __syncthreads();
+        };
+        part_of(std::integral_constant<int, 0>{});
+        if constexpr (H > 1) part_of(std::integral_constant<int, 1>{});
+        if constexpr (H > 2) part_of(std::integral_constant<int, 2>{});
+    }
+    if (ng > 0) post(ibeg + 16 * (ng - 1));
+    if (accumulate) return;
+    // degrees not reached by the step loop: before ibeg (negligible functions) and after nsteps
+    for (int ii = threadIdx.x; ii < nsteps_out; ii += NT) {
+        if (ii >= ibeg && ii < ibeg + 16 * ng) continue;
+        const int le = o.mfun + 2 * ii;
+        for (int f = fbase; f < min(nfields, fbase + 4 * CT); ++f) {
+            double2 *Qf = Qbase + (size_t)f * spec_dist;
+            if (le <= spec_ltop) Qf[le] = make_double2(0.0, 0.0);
+            if (le + 1 <= spec_ltop) Qf[le + 1] = make_double2(0.0, 0.0);
+        }
+    }
+    if (vector_mode && im == 0 && threadIdx.x == 0)   // degree 0 of the vector m=0 spectra
+        for (int f = fbase; f < min(nfields, fbase + 4 * CT); ++f) Qbase[(size_t)f * spec_dist] = make_double2(0.0, 0.0);
+}
+
+template <int NTB, int CT, int TT, int H, int PREC>
+void launch_anal_shared(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
+                        int spec_ltop, hipStream_t s, int tile_base, int tiles, int accumulate) {
+    const DeviceTables *t = a.t;
+    dim3 grid((a.mmax + 1) * ((a.nfields + 4 * CT - 1) / (4 * CT)));
+    hipLaunchKernelGGL((legendre_anal_shared_kernel<NTB, CT, TT, H, PREC>), grid, dim3(64 * CT * TT), 0, s, t->x, t->x2,
+                       t->wq, t->step_ofs, t->ab, t->pm, a.vector_mode ? t->i0v : t->i0, a.vector_mode ? t->z0v : t->z0,
+                       F, four_dist, Q, spec_dist, spec_ltop == a.lmax + 1 ? a.lmax + 1 : a.lmax, spec_ltop, a.mmax,
+                       a.mres, a.nlat, a.nlat_2, a.ltr, a.imlim, a.nfields, a.vector_mode, a.mpos_scale, a.lat_weight,
+                       tile_base, std::min(a.nlat_2, (tile_base + tiles) * 64), accumulate);
+}
+
 // Q[f][i] = sum_s part[s][f][i], i < n (the latitude splits' partial spectra)
 void launch_sum_splits(const double2 *part, long part_dist, int nsplit, int nfields, double2 *Q, long spec_dist,
                        long n, hipStream_t s);
 
-template <int PREC>
-void anal_launch(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
-                 int spec_ltop, hipStream_t s) {
+// One or two fields in FP64 (4x4x4 blocks, no idle matrix-core columns).
+inline void anal_launch_few(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
+                            int spec_ltop, hipStream_t s) {
     const int ntiles = (a.nlat_2 + 63) / 64;
-    if constexpr (PREC == 0) {
-        const int ns = anal_splits(a);
-        if (ns > 1 && a.part) {   // 12-wave blocks over a latitude split each, then the sum
-            for (int k = 0; k < ns; ++k) {
-                double2 *P = a.part + (size_t)k * a.nfields * a.part_dist;
-                // one field: two 16-step groups per barrier round where the coefficient table
-                // still fits in LDS beside the larger partial-tile buffer
-                if (a.nfields == 1 && anal_cf_fits(anal_static_lds(12, 1, 4, 2), a.ltr))
-                    launch_anal_t<12, 1, 1, 0, 1, 1, 2>(a, F, four_dist, P, a.part_dist, spec_ltop, s, 12 * k);
-                else if (a.nfields == 1) launch_anal_t<12, 1, 1, 0, 1>(a, F, four_dist, P, a.part_dist, spec_ltop, s, 12 * k);
-                else launch_anal_t<12, 1, 1, 0, 2>(a, F, four_dist, P, a.part_dist, spec_ltop, s, 12 * k);
-            }
-            launch_sum_splits(a.part, a.part_dist, ns, a.nfields, Q, spec_dist, a.part_dist, s);
-            return;
+    const int ns = anal_splits(a);
+    if (ns > 1 && a.part) {   // 12-wave blocks over a latitude split each, then the sum
+        for (int k = 0; k < ns; ++k) {
+            double2 *P = a.part + (size_t)k * a.nfields * a.part_dist;
+            // one field: two 16-step groups per barrier round where the coefficient table
+            // still fits in LDS beside the larger partial-tile buffer
+            if (a.nfields == 1 && anal_cf_fits(anal_static_lds(12, 1, 2), a.ltr))
+                launch_anal_few<12, 1, 1, 2>(a, F, four_dist, P, a.part_dist, spec_ltop, s, 12 * k);
+            else if (a.nfields == 1) launch_anal_few<12, 1, 1>(a, F, four_dist, P, a.part_dist, spec_ltop, s, 12 * k);
+            else launch_anal_few<12, 1, 2>(a, F, four_dist, P, a.part_dist, spec_ltop, s, 12 * k);
         }
+        launch_sum_splits(a.part, a.part_dist, ns, a.nfields, Q, spec_dist, a.part_dist, s);
+        return;
     }
     // waves per block: one latitude tile per wave up to 12 waves (measured fastest: lowest
     // register count, 3 waves per SIMD); beyond, a divisor of the tile count, at most 8
@@ -876,28 +1208,10 @@ void anal_launch(const LegendreArgs &a, const double2 *F, long four_dist, double
     if (a.anal_nw > 0 && ntiles % a.anal_nw == 0 && anal_shape_ok(a.anal_nw, ntiles / a.anal_nw)) nw = a.anal_nw;
     int nlr = ntiles / nw;
     if (nlr > 6) { nw = 8; nlr = (ntiles + 7) / 8; }
-    static const int ncg_env = getenv("SHTNS_AMD_ANAL_NCG") ? atoi(getenv("SHTNS_AMD_ANAL_NCG")) : 0;
-    const int ncg_want = a.anal_ncg ? a.anal_ncg : ncg_env;
-    bool wide = (a.nfields > 4) && (nlr <= 3);   // 8 fields per block when registers allow
-    if (ncg_want == 1) wide = false;
-    if (ncg_want == 2 && nlr <= 3) wide = (a.nfields > 4);
-    // one or two fields (FP64): 4x4x4 blocks, no idle matrix-core columns
-    const int nf4 = (PREC == 0 && a.nfields <= 2 && !synth_force16()) ? a.nfields : 0;
-    // six one-tile waves and more than one 8-field group: two groups per block, 12 waves (three
-    // on every SIMD instead of 1.5); SHTNS_AMD_ANAL_NG=1 keeps the 6-wave blocks
-    static const int ng_env = getenv("SHTNS_AMD_ANAL_NG") ? atoi(getenv("SHTNS_AMD_ANAL_NG")) : 0;
-    if (nf4 == 0 && nw == 6 && nlr == 1 && wide && a.nfields > 8 && ng_env != 1) {
-        launch_anal_t<6, 1, 2, PREC, 0, 2>(a, F, four_dist, Q, spec_dist, spec_ltop, s);
-        return;
-    }
 #define ANAL_CASE(W, R)                                                                              \
     if (nw == W && nlr <= R) {                                                                       \
-        if constexpr (PREC == 0) {                                                                   \
-            if (nf4 == 1) { launch_anal_t<W, R, 1, 0, 1>(a, F, four_dist, Q, spec_dist, spec_ltop, s); return; } \
-            if (nf4 == 2) { launch_anal_t<W, R, 1, 0, 2>(a, F, four_dist, Q, spec_dist, spec_ltop, s); return; } \
-        }                                                                                            \
-        if (wide) launch_anal_t<W, R, 2, PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s);        \
-        else launch_anal_t<W, R, 1, PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s);             \
+        if (a.nfields == 1) launch_anal_few<W, R, 1>(a, F, four_dist, Q, spec_dist, spec_ltop, s);   \
+        else launch_anal_few<W, R, 2>(a, F, four_dist, Q, spec_dist, spec_ltop, s);                  \
         return;                                                                                      \
     }
     ANAL_CASE(1, 1) ANAL_CASE(1, 2) ANAL_CASE(1, 3) ANAL_CASE(1, 6)
@@ -911,6 +1225,63 @@ void anal_launch(const LegendreArgs &a, const double2 *F, long four_dist, double
     ANAL_CASE(9, 1) ANAL_CASE(10, 1) ANAL_CASE(11, 1) ANAL_CASE(12, 1)
 #undef ANAL_CASE
     fprintf(stderr, "shtns_amd: no analysis kernel for nlat_2=%d\n", a.nlat_2);
+}
+
+// Block shape (tiles, column tiles, parts, halves) of the shared kernel for a number of latitude
+// tiles (rounded up to a compiled one) and ctn column tiles of 4 fields.  Measured on FP64
+// batches (analysis call with its FFT, us; the one-group kernel it replaced, other shapes):
+//   lmax  127,  8 / 32 fields: (2,1,4) 22.5 / 30.2   [28.9 / 36.5; (2,2,2) 25.2 / 32.4]
+//   lmax  255,  8 / 16 fields: (3,1,4) 36.6 / 46.1   [43.1 / 52.7; (3,2,2) 41.0 / 50.1]
+//               32 fields:     (3,2,2) 69.0          [82.6; (3,1,4) 72.6, (3,4,2) 73.0]
+//   lmax  340, 32 fields:      (4,2,4) 115           [(4,2,2) 120, (4,1,4) 123]
+//   lmax  511,  8 / 16 fields: (6,2,4) 92 / 162      [100 / 170; (6,4,3) 121 / 170, (6,2,2) 104 / 183]
+//               64 fields:     (6,2,4) 591           [(6,4,3) 650, (6,2,2) 653, (6,2,3) 945]
+//   lmax  680,  8 / 16 fields: (8,2,4) 230, (8,4,2) 435   [- / 451; (8,1,4) 294 / 594]
+//   lmax 1023,  4 / 8 / 16:    (12,1,4,3) 303, (12,2,6) 488, (12,4,3) 885   [310 / 504 / 990]
+// Two blocks of eight waves per CU overlap one block's recurrence, loads and barriers with the
+// other's contraction where their LDS allows ((6,2,4)); at 12 tiles the recurrence buffer
+// leaves one block per CU, and more fields per block amortize those phases.  Six-wave blocks
+// load two of the four SIMDs twice.  With few columns, four waves share an order (latency).
+// One and two tiles are split by half tiles, which sums in the order of the one- and two-field
+// kernel: there a field's result does not depend on its batch.
+template <int PREC>
+void anal_launch_shared(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
+                        int spec_ltop, hipStream_t s) {
+    const int ntiles = (a.nlat_2 + 63) / 64, ns = (ntiles + 11) / 12, per = (ntiles + ns - 1) / ns;
+    const int ctn = (a.nfields + 3) / 4;
+    // the tuner's choice: 1 for four fields per block, otherwise as many as the shapes below take
+    static const int ncg_env = getenv("SHTNS_AMD_ANAL_NCG") ? atoi(getenv("SHTNS_AMD_ANAL_NCG")) : 0;
+    const bool one = (a.anal_ncg ? a.anal_ncg : ncg_env) == 1;
+    for (int k = 0; k < ns; ++k) {   // in order on the stream: the later splits add to the first one's result
+#define ANAL_SHARED(...) launch_anal_shared<__VA_ARGS__, PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s, k * per, per, k > 0)
+        if (per <= 1) { if (ctn >= 2 && !one) ANAL_SHARED(1, 2, 2, 1); else ANAL_SHARED(1, 1, 2, 1); }
+        else if (per <= 2) ANAL_SHARED(2, 1, 4, 1);
+        else if (per <= 3) { if (ctn > 4 && !one) ANAL_SHARED(3, 2, 2, 1); else ANAL_SHARED(3, 1, 4, 1); }
+        else if (per <= 4) { if (ctn > 4 && !one) ANAL_SHARED(4, 2, 4, 1); else ANAL_SHARED(4, 1, 4, 1); }
+        else if (per <= 6) { if (ctn >= 2 && !one) ANAL_SHARED(6, 2, 4, 1); else ANAL_SHARED(6, 1, 4, 1); }
+        else if (per <= 8) {
+            if (ctn >= 3 && !one) ANAL_SHARED(8, 4, 2, 1);
+            else if (ctn >= 2 && !one) ANAL_SHARED(8, 2, 4, 1);
+            else ANAL_SHARED(8, 1, 4, 1);
+        } else {
+            if (ctn >= 3 && !one) ANAL_SHARED(12, 4, 3, 1);
+            else if (ctn >= 2 && !one) ANAL_SHARED(12, 2, 6, 1);
+            else ANAL_SHARED(12, 1, 4, 3);
+        }
+#undef ANAL_SHARED
+    }
+}
+
+template <int PREC>
+void anal_launch(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
+                 int spec_ltop, hipStream_t s) {
+    if constexpr (PREC == 0) {
+        if (a.nfields <= 2 && !synth_force16()) {
+            anal_launch_few(a, F, four_dist, Q, spec_dist, spec_ltop, s);
+            return;
+        }
+    }
+    anal_launch_shared<PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s);
 }
 
 }  // namespace shtns_amd
