@@ -1252,17 +1252,31 @@ void anal_launch_shared(const LegendreArgs &a, const double2 *F, long four_dist,
     // the tuner's choice: 1 for four fields per block, otherwise as many as the shapes below take
     static const int ncg_env = getenv("SHTNS_AMD_ANAL_NCG") ? atoi(getenv("SHTNS_AMD_ANAL_NCG")) : 0;
     const bool one = (a.anal_ncg ? a.anal_ncg : ncg_env) == 1;
+    if (per > 6 && ctn > 4 && (ctn % 4 == 1 || ctn % 4 == 2) && !one) {
+        // shapes of 16 fields: the last one to eight fields in blocks of their own size (in the
+        // 16-field blocks their waves would wait for nothing: 24 fields at lmax=850 1462 us)
+        const int nf0 = (ctn & ~3) * 4;
+        LegendreArgs a0 = a, a1 = a;
+        a0.nfields = nf0;
+        a1.nfields = a.nfields - nf0;
+        anal_launch_shared<PREC>(a0, F, four_dist, Q, spec_dist, spec_ltop, s);
+        anal_launch_shared<PREC>(a1, F + (size_t)nf0 * four_dist, four_dist, Q + (size_t)nf0 * spec_dist, spec_dist, spec_ltop, s);
+        return;
+    }
     for (int k = 0; k < ns; ++k) {   // in order on the stream: the later splits add to the first one's result
 #define ANAL_SHARED(...) launch_anal_shared<__VA_ARGS__, PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s, k * per, per, k > 0)
         if (per <= 1) { if (ctn >= 2 && !one) ANAL_SHARED(1, 2, 2, 1); else ANAL_SHARED(1, 1, 2, 1); }
         else if (per <= 2) ANAL_SHARED(2, 1, 4, 1);
         else if (per <= 3) { if (ctn > 4 && !one) ANAL_SHARED(3, 2, 2, 1); else ANAL_SHARED(3, 1, 4, 1); }
-        else if (per <= 4) { if (ctn > 4 && !one) ANAL_SHARED(4, 2, 4, 1); else ANAL_SHARED(4, 1, 4, 1); }
-        else if (per <= 6) { if (ctn >= 2 && !one) ANAL_SHARED(6, 2, 4, 1); else ANAL_SHARED(6, 1, 4, 1); }
-        else if (per <= 8) {
+        else if (per <= 4) { if (ctn >= 4 && !one) ANAL_SHARED(4, 2, 4, 1); else ANAL_SHARED(4, 1, 4, 1); }
+        else if (per <= 6) {
+            if (ctn >= 2 && !one) ANAL_SHARED(6, 2, 4, 1);
+            else if (per == 6) ANAL_SHARED(6, 1, 4, 1);
+            else ANAL_SHARED(5, 1, 5, 1);
+        } else if (per <= 8) {
             if (ctn >= 3 && !one) ANAL_SHARED(8, 4, 2, 1);
             else if (ctn >= 2 && !one) ANAL_SHARED(8, 2, 4, 1);
-            else ANAL_SHARED(8, 1, 4, 1);
+            else ANAL_SHARED(8, 1, 8, 1);
         } else {
             if (ctn >= 3 && !one) ANAL_SHARED(12, 4, 3, 1);
             else if (ctn >= 2 && !one) ANAL_SHARED(12, 2, 6, 1);
