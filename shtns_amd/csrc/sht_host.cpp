@@ -445,6 +445,24 @@ extern "C" void shtns_free(void *p) {
 // ------------------------------------------------------------------------------------------
 // grid
 // ------------------------------------------------------------------------------------------
+// Radices of the in-place FFT of M points: 4, 2, 3, 5, 7 in this order for the lengths whose
+// kernels are specialized on it; otherwise the fewest passes of the runtime-plan kernel's
+// radices, powers of two first (the last pass' short spacing then has an odd radix, which
+// spreads over the LDS banks).
+static void best_radices(int n, int from, std::vector<int> &cur, std::vector<int> &best) {
+    static const int order[] = {16, 8, 12, 4, 10, 6, 2, 15, 9, 5, 3, 7};
+    if (n == 1) {
+        if (best.empty() || cur.size() < best.size()) best = cur;
+        return;
+    }
+    if (!best.empty() && cur.size() + 1 >= best.size()) return;
+    for (int k = from; k < 12; ++k) {
+        if (n % order[k]) continue;
+        cur.push_back(order[k]);
+        best_radices(n / order[k], k, cur, best);
+        cur.pop_back();
+    }
+}
 static int factor_fft(int M, FftPlan &plan) {
     plan.M = M;
     plan.nstages = 0;
@@ -453,7 +471,14 @@ static int factor_fft(int M, FftPlan &plan) {
     const int small[] = {2, 3, 5, 7};
     for (int p : small)
         while (n % p == 0 && plan.nstages < 24) { plan.radix[plan.nstages++] = p; n /= p; }
-    return (n == 1) ? 0 : -1;
+    if (n != 1) return -1;
+    if (!lds_fft_specialized(M)) {
+        std::vector<int> cur, best;
+        best_radices(M, 0, cur, best);
+        plan.nstages = (int)best.size();
+        for (size_t k = 0; k < best.size(); ++k) plan.radix[k] = best[k];
+    }
+    return 0;
 }
 
 // digit-reversal: position of bin k after the in-place DIF stages of `plan`

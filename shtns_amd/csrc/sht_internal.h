@@ -247,6 +247,18 @@ bool launch_fft_synth_coop(const DeviceTables *t, int nlat, int M, int imlim, in
 bool launch_fft_anal_coop(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const double *V,
                           long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
                           int lat_end, int nthreads = 256);
+// any length (t->plan, t->fft_pos), runtime plan in LDS (sht_fft_any.hip); false when the length
+// does not fit a CU's LDS
+bool launch_fft_synth_any(const DeviceTables *t, int nlat, int imlim, int nfields, const double2 *F, long four_dist,
+                          double *V, long spat_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end);
+bool launch_fft_synth_any(const DeviceTables *t, int nlat, int imlim, int nfields, const double2 *F, long four_dist,
+                          float *V, long spat_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end);
+bool launch_fft_anal_any(const DeviceTables *t, int nlat, int mmax, int imlim, int nfields, const double *V,
+                         long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
+                         int lat_end);
+bool launch_fft_anal_any(const DeviceTables *t, int nlat, int mmax, int imlim, int nfields, const float *V,
+                         long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
+                         int lat_end);
 bool lds_fft_specialized(int M);   // an LDS-staged FFT kernel compiled for this length
 // raise a kernel's dynamic LDS limit once (outside any launch sequence that may be captured)
 void ensure_lds_limit(const void *kern, size_t lds);

@@ -921,11 +921,8 @@ void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int mmax, int i
     }
     FFT_SIZES(FFT_SYN_CASE)
 #undef FFT_SYN_CASE
-    const int T = fft_lat_per_block(M);
-    const size_t lds = (size_t)T * M * sizeof(double2);
-    set_lds_limit(fft_synth_kernel<0, 1>, lds);
-    hipLaunchKernelGGL((fft_synth_kernel<0, 1>), dim3((nlat_chunk + T - 1) / T, nfields), dim3(256), lds, s, F,
-                       four_dist, V, spat_dist, t->roots, t->fft_pos, t->plan, nlat, imlim, sp, st, T, lat_base, lat_end);
+    if (!launch_fft_synth_any(t, nlat, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end))
+        set_error(2, "no longitude FFT for nphi=%d", nphi);
     (void)mmax;
 }
 
@@ -979,12 +976,8 @@ void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int im
     }
     FFT_SIZES(FFT_ANA_CASE)
 #undef FFT_ANA_CASE
-    const int T = fft_lat_per_block(M);
-    const size_t lds = (size_t)T * M * sizeof(double2);
-    set_lds_limit(fft_anal_kernel<0, 1>, lds);
-    hipLaunchKernelGGL((fft_anal_kernel<0, 1>), dim3((nlat_chunk + T - 1) / T, nfields), dim3(256), lds, s, V,
-                       spat_dist, F, four_dist, t->roots, t->fft_pos, t->plan, nlat, mmax, imlim, sp, st, T, lat_base,
-                       lat_end);
+    if (!launch_fft_anal_any(t, nlat, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base, lat_end))
+        set_error(2, "no longitude FFT for nphi=%d", nphi);
 }
 
 // ---------------------------------------------------------------------------------------
