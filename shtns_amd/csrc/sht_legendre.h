@@ -150,7 +150,17 @@ struct Contract {
 // The accumulators go straight to F: lanes holding E and O of one field are lane^2
 // partners (north = E + x O, south = E - x O).
 // ---------------------------------------------------------------------------------------
-constexpr int kSynthWaves = 4;
+constexpr int kSynthTileBytes = 2 * 4 * 64 * sizeof(double);   // LDS per wave
+// Waves (latitude tiles) per block.  Blocks of four waves whose last ones have no tile leave
+// their SIMDs idle: with six tiles half of the blocks loaded two SIMDs only (matrix cores busy
+// 54%; 32 vector pairs at lmax=511: Legendre synthesis 358 -> 305 us in one-wave blocks), so
+// other counts than multiples of four take one-wave blocks (lmax=560, 16 fields: call 257 ->
+// 243 us; two-wave ones 257).  One to three fields are bound by latency and keep an order's
+// tiles together (lmax=340, 3 fields: 41.5 us, one-wave blocks 44.3).
+inline int synth_waves(int ntl, int nfields) {
+    if (nfields <= 3) return ntl < 4 ? ntl : 4;
+    return ntl % 4 == 0 ? 4 : ntl == 2 ? 2 : 1;
+}
 
 // NF4 > 0 (FP64, NCG = 1, at most 3 fields): field c of the group is contracted with
 // v_mfma_f64_4x4x4f64 (four 4x4x4 blocks: 16 latitudes x 4 steps x the field's 4 columns),
@@ -166,16 +176,18 @@ __global__ __launch_bounds__(256) void legendre_synth_kernel(
     int nsteps_total, int lmax_spec, double2 *__restrict__ F, long four_dist, int mmax, int mres, int nlat,
     int nlat_2, int ltr, int imlim, int nfields, int vector_mode, int lat_weight, int tile0, int ntl) {
     constexpr int NCOL = 16 * NCG;
-    __shared__ double ytile[kSynthWaves][2][4][64];
+    extern __shared__ double ytile_lds[];   // [waves][2][4][64]
+    double(*ytile)[2][4][64] = reinterpret_cast<double(*)[2][4][64]>(ytile_lds);
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     // heavy orders first: block x -> (order, tile group); the tile groups of one order run on
     // one XCD (they read the same coefficient rows, which then hit in that XCD's L2)
-    const int ntg = (ntl + kSynthWaves - 1) / kSynthWaves;   // tile groups of this launch
+    const int nw = blockDim.x >> 6;
+    const int ntg = (ntl + nw - 1) / nw;   // tile groups of this launch
     const int bx = xcd_cluster(blockIdx.x, gridDim.x, ntg);
     const int im = bx / ntg;
-    const int tile = tile0 + (bx - im * ntg) * kSynthWaves + wave;
+    const int tile = tile0 + (bx - im * ntg) * nw + wave;
     const int g = blockIdx.y;
     const int fbase = g * 4 * NCG;
     if (tile >= tile0 + ntl || tile * 64 >= nlat_2) return;   // no block-level synchronization in this kernel
@@ -412,12 +424,13 @@ template <int PREC>
 void synth_tiles_launch(const LegendreArgs &a, int spec_ltop, double2 *F, long four_dist, const double *qmix,
                         int nsteps_total, int tile0, int ntl, hipStream_t s) {
     const DeviceTables *t = a.t;
-    const int ntg = (ntl + kSynthWaves - 1) / kSynthWaves;
+    const int nw = synth_waves(ntl, a.nfields);
+    const int ntg = (ntl + nw - 1) / nw;
     const int ncg = synth_ncg(a.nfields, a.synth_ncg);
     const int ng = (a.nfields + 4 * ncg - 1) / (4 * ncg);
     dim3 grid((a.mmax + 1) * ntg, ng);
 #define SYNTH_LAUNCH(NC, ...)                                                                                    \
-    hipLaunchKernelGGL((legendre_synth_kernel<NC, PREC, ##__VA_ARGS__>), grid, dim3(64 * kSynthWaves), 0, s, t->x, t->x2, t->st, t->wq, \
+    hipLaunchKernelGGL((legendre_synth_kernel<NC, PREC, ##__VA_ARGS__>), grid, dim3(64 * nw), nw * kSynthTileBytes, s, t->x, t->x2, t->st, t->wq, \
                        t->step_ofs, t->ab, a.vector_mode ? t->i0v : t->i0, a.vector_mode ? t->z0v : t->z0, qmix, \
                        nsteps_total, spec_ltop, F, four_dist, a.mmax,                                              \
                        a.mres, a.nlat, a.nlat_2, a.ltr, a.imlim, a.nfields, a.vector_mode, a.lat_weight, tile0, ntl)
