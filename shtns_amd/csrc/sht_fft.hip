@@ -514,9 +514,9 @@ struct CoopSGeom {
 // those of the doubles of the complex array).  gridDim.x is twice the latitude groups, and
 // the part is bit 3 of the block index: blocks b and b + 8 run on the same XCD, one after
 // the other, and write the two halves of the same cache lines, which merge in that L2.
-template <int M, int NTB>
+template <int M, int NTB, class TV>
 __global__ __launch_bounds__(NTB) void fft_synth_coops(const double2 *__restrict__ F, long four_dist,
-                                                       double *__restrict__ V, long spat_dist,
+                                                       TV *__restrict__ V, long spat_dist,
                                                        const double2 *__restrict__ roots, int nlat, int imlim,
                                                        long sp, long stt, int lat_base, int lat_end, long fpart) {
     using CG = CoopSGeom<M, NTB>;
@@ -575,15 +575,16 @@ __global__ __launch_bounds__(NTB) void fft_synth_coops(const double2 *__restrict
     seq_sync<M>();
     wave_passes_split<M, 1, 0>(v, seq, l, roots);
     // z_n out: real parts to rows 2n, then imaginary parts to rows 2n+1
-    const unsigned off = 8u * (unsigned)((live ? lat0 + tl : 0) * stt + 2 * row * sp);
-    const unsigned step = 8u * (unsigned)(2 * ROWS * sp), odd = 8u * (unsigned)sp;
-    double *Vf = V + (size_t)blockIdx.y * spat_dist + part;
+    constexpr unsigned SV = sizeof(TV);
+    const unsigned off = SV * (unsigned)((live ? lat0 + tl : 0) * stt + 2 * row * sp);
+    const unsigned step = SV * (unsigned)(2 * ROWS * sp), odd = SV * (unsigned)sp;
+    TV *Vf = V + (size_t)blockIdx.y * spat_dist + part;
     sfor<R>([&](auto jc) { seq[slot_at<LQ>(l, decltype(jc)::value)] = v[decltype(jc)::value].x; });
     __syncthreads();
     if (live)
         sfor<R>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            at(Vf, off + i * step) = mine[slot_at<ROWS>(row, i)];
+            at(Vf, off + i * step) = (TV)mine[slot_at<ROWS>(row, i)];
         });
     __syncthreads();
     sfor<R>([&](auto jc) { seq[slot_at<LQ>(l, decltype(jc)::value)] = v[decltype(jc)::value].y; });
@@ -591,14 +592,14 @@ __global__ __launch_bounds__(NTB) void fft_synth_coops(const double2 *__restrict
     if (live)
         sfor<R>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            at(Vf, off + i * step + odd) = mine[slot_at<ROWS>(row, i)];
+            at(Vf, off + i * step + odd) = (TV)mine[slot_at<ROWS>(row, i)];
         });
 }
 
 // With 256 threads (52 KB of LDS at M = 1536) three blocks fit in a CU's LDS; the register
 // budget of three waves per SIMD (168 VGPRs) lets them all be resident.
-template <int M, int NTB>
-__global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB == 256 ? 3 : 1))) void fft_anal_coops(const double *__restrict__ V, long spat_dist,
+template <int M, int NTB, class TV>
+__global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB == 256 ? 3 : 1))) void fft_anal_coops(const TV *__restrict__ V, long spat_dist,
                                                       double2 *__restrict__ F, long four_dist,
                                                       const double2 *__restrict__ roots, int nlat, int mmax,
                                                       int imlim, long sp, long stt, int lat_base, int lat_end,
@@ -623,13 +624,14 @@ __global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB == 256 
     // z_n = V[2n] + i V[2n+1] of the block's latitudes, latitude fastest
     double zx[R], zy[R];
     {
-        const double *Vf = V + (size_t)blockIdx.y * spat_dist + part;
-        const unsigned off = 8u * (unsigned)((live ? lat0 + tl : 0) * stt + 2 * row * sp);
-        const unsigned step = 8u * (unsigned)(2 * ROWS * sp), odd = 8u * (unsigned)sp;
+        constexpr unsigned SV = sizeof(TV);
+        const TV *Vf = V + (size_t)blockIdx.y * spat_dist + part;
+        const unsigned off = SV * (unsigned)((live ? lat0 + tl : 0) * stt + 2 * row * sp);
+        const unsigned step = SV * (unsigned)(2 * ROWS * sp), odd = SV * (unsigned)sp;
         sfor<R>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
-            zx[i] = live ? at(Vf, off + i * step) : 0.0;
-            zy[i] = live ? at(Vf, off + i * step + odd) : 0.0;
+            zx[i] = live ? (double)at(Vf, off + i * step) : 0.0;
+            zy[i] = live ? (double)at(Vf, off + i * step + odd) : 0.0;
         });
     }
     sfor<R>([&](auto ic) { mine[slot_at<ROWS>(row, decltype(ic)::value)] = zx[decltype(ic)::value]; });
@@ -807,19 +809,19 @@ bool anal_coop(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int 
     return false;
 }
 
-template <int NTB>
+template <int NTB, class TV>
 bool synth_coops(const DeviceTables *t, int nlat, int M, int imlim, int nfields, const double2 *F, long four_dist,
-                 double *V, long spat_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end,
+                 TV *V, long spat_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end,
                  long fpart = 0, bool dry = false) {
 #define SYN_COOPS(MM)                                                                                         \
     if (M == MM) {                                                                                            \
         using CG = CoopSGeom<MM, NTB>;                                                                        \
         static_assert(CG::LQ <= 64 && CG::T >= 2 && CG::T * CG::LQ == CG::NT, "cooperative FFT shape");      \
-        lds_limit(fft_synth_coops<MM, NTB>, CG::lds_bytes);                                                   \
+        lds_limit(fft_synth_coops<MM, NTB, TV>, CG::lds_bytes);                                                   \
         const int nb = (lat_end - lat_base + CG::T - 1) / CG::T;                                             \
         if (fpart > 0 && nb % 8) return false;   /* the part / XCD decoding needs whole groups of 8 */        \
         if (dry) return true;                                                                                 \
-        hipLaunchKernelGGL((fft_synth_coops<MM, NTB>), dim3(fpart > 0 ? 2 * nb : nb, nfields), dim3(CG::NT),  \
+        hipLaunchKernelGGL((fft_synth_coops<MM, NTB, TV>), dim3(fpart > 0 ? 2 * nb : nb, nfields), dim3(CG::NT),  \
                            CG::lds_bytes, s, F, four_dist, V, spat_dist, t->roots, nlat, imlim, sp, st,       \
                            lat_base, lat_end, fpart);                                                         \
         return true;                                                                                          \
@@ -829,18 +831,18 @@ bool synth_coops(const DeviceTables *t, int nlat, int M, int imlim, int nfields,
     return false;
 }
 
-template <int NTB>
-bool anal_coops(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const double *V,
+template <int NTB, class TV>
+bool anal_coops(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const TV *V,
                 long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end,
                 long fpart = 0, bool dry = false) {
 #define ANA_COOPS(MM)                                                                                         \
     if (M == MM) {                                                                                            \
         using CG = CoopSGeom<MM, NTB>;                                                                        \
-        lds_limit(fft_anal_coops<MM, NTB>, CG::lds_bytes);                                                    \
+        lds_limit(fft_anal_coops<MM, NTB, TV>, CG::lds_bytes);                                                    \
         const int nb = (lat_end - lat_base + CG::T - 1) / CG::T;                                             \
         if (fpart > 0 && nb % 8) return false;   /* the part / XCD decoding needs whole groups of 8 */        \
         if (dry) return true;                                                                                 \
-        hipLaunchKernelGGL((fft_anal_coops<MM, NTB>), dim3(fpart > 0 ? 2 * nb : nb, nfields), dim3(CG::NT),   \
+        hipLaunchKernelGGL((fft_anal_coops<MM, NTB, TV>), dim3(fpart > 0 ? 2 * nb : nb, nfields), dim3(CG::NT),   \
                            CG::lds_bytes, s, V, spat_dist, F, four_dist, t->roots, nlat, mmax, imlim, sp, st, \
                            lat_base, lat_end, fpart);                                                         \
         return true;                                                                                          \
@@ -864,9 +866,9 @@ bool launch_fft_synth_coop(const DeviceTables *t, int nlat, int M, int imlim, in
                            int lat_end, int nthreads) {
     if (!coop_offsets_fit(nlat, M, imlim, sp, st)) return false;
     if (nthreads == -256)
-        return synth_coops<256>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
+        return synth_coops<256, double>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
     if (nthreads == -512)
-        return synth_coops<512>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
+        return synth_coops<512, double>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
     if (nthreads == 128)
         return synth_coop<128>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
     return synth_coop<256>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
@@ -877,9 +879,9 @@ bool launch_fft_synth_coops_pairs(const DeviceTables *t, int nlat, int M, int im
                                   int nthreads, bool dry) {
     if (fpart <= 0 || !coop_offsets_fit(nlat, M, imlim, sp, st)) return false;
     if (nthreads == -512)
-        return synth_coops<512>(t, nlat, M, imlim, nf, F, fdist, V, spat_dist, sp, st, s, 0, nlat, fpart, dry);
+        return synth_coops<512, double>(t, nlat, M, imlim, nf, F, fdist, V, spat_dist, sp, st, s, 0, nlat, fpart, dry);
     if (nthreads == -256)
-        return synth_coops<256>(t, nlat, M, imlim, nf, F, fdist, V, spat_dist, sp, st, s, 0, nlat, fpart, dry);
+        return synth_coops<256, double>(t, nlat, M, imlim, nf, F, fdist, V, spat_dist, sp, st, s, 0, nlat, fpart, dry);
     return false;
 }
 
@@ -888,9 +890,9 @@ bool launch_fft_anal_coops_pairs(const DeviceTables *t, int nlat, int M, int mma
                                  int nthreads, bool dry) {
     if (fpart <= 0 || !coop_offsets_fit(nlat, M, std::max(mmax, imlim), sp, st)) return false;
     if (nthreads == -512)
-        return anal_coops<512>(t, nlat, M, mmax, imlim, nf, V, spat_dist, F, fdist, sp, st, s, 0, nlat, fpart, dry);
+        return anal_coops<512, double>(t, nlat, M, mmax, imlim, nf, V, spat_dist, F, fdist, sp, st, s, 0, nlat, fpart, dry);
     if (nthreads == -256)
-        return anal_coops<256>(t, nlat, M, mmax, imlim, nf, V, spat_dist, F, fdist, sp, st, s, 0, nlat, fpart, dry);
+        return anal_coops<256, double>(t, nlat, M, mmax, imlim, nf, V, spat_dist, F, fdist, sp, st, s, 0, nlat, fpart, dry);
     return false;
 }
 
@@ -899,10 +901,10 @@ bool launch_fft_anal_coop(const DeviceTables *t, int nlat, int M, int mmax, int 
                           int lat_end, int nthreads) {
     if (!coop_offsets_fit(nlat, M, std::max(mmax, imlim), sp, st)) return false;
     if (nthreads == -256)
-        return anal_coops<256>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
+        return anal_coops<256, double>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
                                lat_end);
     if (nthreads == -512)
-        return anal_coops<512>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
+        return anal_coops<512, double>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
                                lat_end);
     if (nthreads == 128)
         return anal_coop<128>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
@@ -923,6 +925,18 @@ bool launch_fft_anal_wave(const DeviceTables *t, int nlat, int M, int mmax, int 
                           long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
                           int lat_end) {
     return anal_wave(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base, lat_end);
+}
+
+// single-precision fields, 256 threads
+bool launch_fft_synth_coops_f32(const DeviceTables *t, int nlat, int M, int imlim, int nfields, const double2 *F,
+                                long four_dist, float *V, long spat_dist, long sp, long st, hipStream_t s) {
+    if (!coop_offsets_fit(nlat, M, imlim, sp, st)) return false;
+    return synth_coops<256, float>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat);
+}
+bool launch_fft_anal_coops_f32(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const float *V,
+                               long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s) {
+    if (!coop_offsets_fit(nlat, M, std::max(mmax, imlim), sp, st)) return false;
+    return anal_coops<256, float>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat);
 }
 
 }  // namespace shtns_amd

@@ -229,22 +229,22 @@ template <class TV>
 bool synth_any(const DeviceTables *t, int nlat, int imlim, int nfields, const double2 *F, long four_dist, TV *V,
                long spat_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end) {
     AnyGeom g;
-    if (!any_geom(t->plan, lat_end - lat_base, nfields, g)) return false;
+    if (!any_geom(t->any_plan, lat_end - lat_base, nfields, g)) return false;
     ensure_lds_limit((const void *)fft_synth_any<TV>, g.lds);
     const int nb = (lat_end - lat_base + (1 << g.lt) - 1) >> g.lt;
     hipLaunchKernelGGL(fft_synth_any<TV>, dim3(nb, nfields), dim3(g.nt), g.lds, s, F, four_dist, V, spat_dist, t->roots,
-                       t->fft_pos, g.pl, nlat, imlim, sp, st, g.lt, g.str, lat_base, lat_end);
+                       t->any_pos, g.pl, nlat, imlim, sp, st, g.lt, g.str, lat_base, lat_end);
     return true;
 }
 template <class TV>
 bool anal_any(const DeviceTables *t, int nlat, int mmax, int imlim, int nfields, const TV *V, long spat_dist, double2 *F,
               long four_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end) {
     AnyGeom g;
-    if (!any_geom(t->plan, lat_end - lat_base, nfields, g)) return false;
+    if (!any_geom(t->any_plan, lat_end - lat_base, nfields, g)) return false;
     ensure_lds_limit((const void *)fft_anal_any<TV>, g.lds);
     const int nb = (lat_end - lat_base + (1 << g.lt) - 1) >> g.lt;
     hipLaunchKernelGGL(fft_anal_any<TV>, dim3(nb, nfields), dim3(g.nt), g.lds, s, V, spat_dist, F, four_dist, t->roots,
-                       t->fft_pos, g.pl, nlat, mmax, imlim, sp, st, g.lt, g.str, lat_base, lat_end);
+                       t->any_pos, g.pl, nlat, mmax, imlim, sp, st, g.lt, g.str, lat_base, lat_end);
     return true;
 }
 

@@ -305,7 +305,7 @@ static void free_device(shtns_info *c) {
     (void)hipSetDevice(c->device);
     if (c->clone_of == nullptr) {
         DeviceTables &d = c->d;
-        void *ptrs[] = {d.x, d.x2, d.st, d.wq, d.step_ofs, d.ab, d.pm, d.tm, d.i0, d.z0, d.i0v, d.z0v, d.roots, d.fft_pos,
+        void *ptrs[] = {d.x, d.x2, d.st, d.wq, d.step_ofs, d.ab, d.pm, d.tm, d.i0, d.z0, d.i0v, d.z0v, d.roots, d.fft_pos, d.any_pos,
                         d.sb_ofs, d.eA, d.abk, d.dblk, d.delta, d.nrm};
         for (void *p : ptrs)
             if (p) (void)hipFree(p);
@@ -445,10 +445,8 @@ extern "C" void shtns_free(void *p) {
 // ------------------------------------------------------------------------------------------
 // grid
 // ------------------------------------------------------------------------------------------
-// Radices of the in-place FFT of M points: 4, 2, 3, 5, 7 in this order for the lengths whose
-// kernels are specialized on it; otherwise the fewest passes of the runtime-plan kernel's
-// radices, powers of two first (the last pass' short spacing then has an odd radix, which
-// spreads over the LDS banks).
+// Fewest passes of the runtime-plan FFT's radices for n points, powers of two first (the last
+// pass' short spacing then has an odd radix, which spreads over the LDS banks).
 static void best_radices(int n, int from, std::vector<int> &cur, std::vector<int> &best) {
     static const int order[] = {16, 8, 12, 4, 10, 6, 2, 15, 9, 5, 3, 7};
     if (n == 1) {
@@ -471,14 +469,16 @@ static int factor_fft(int M, FftPlan &plan) {
     const int small[] = {2, 3, 5, 7};
     for (int p : small)
         while (n % p == 0 && plan.nstages < 24) { plan.radix[plan.nstages++] = p; n /= p; }
-    if (n != 1) return -1;
-    if (!lds_fft_specialized(M)) {
-        std::vector<int> cur, best;
-        best_radices(M, 0, cur, best);
-        plan.nstages = (int)best.size();
-        for (size_t k = 0; k < best.size(); ++k) plan.radix[k] = best[k];
-    }
-    return 0;
+    return (n == 1) ? 0 : -1;
+}
+static FftPlan any_fft_plan(int M) {
+    FftPlan plan{};
+    plan.M = M;
+    std::vector<int> cur, best;
+    best_radices(M, 0, cur, best);
+    plan.nstages = (int)best.size();
+    for (size_t k = 0; k < best.size(); ++k) plan.radix[k] = best[k];
+    return plan;
 }
 
 // digit-reversal: position of bin k after the in-place DIF stages of `plan`
@@ -606,6 +606,7 @@ extern "C" int shtns_set_grid_auto(shtns_cfg c, enum shtns_type flags, double ep
         for (unsigned i = 0; i < c->nlat; ++i) c->ct[i] = -c->ct[i];
     c->wg.assign(w.begin(), w.begin() + c->nlat_2);
     c->d.plan = plan;
+    c->d.any_plan = any_fft_plan(plan.M);
     polar_optimize(c, eps);
 
     // GPU tables (a config is usable for queries without a GPU; transforms then fail)
@@ -1026,11 +1027,14 @@ static int device_init(shtns_info *c) {
     }
     std::vector<int> pos;
     fft_positions(d.plan, pos);
+    std::vector<int> any_pos;
+    fft_positions(d.any_plan, any_pos);
 
     if (upload(&d.x, x.data(), nl2) || upload(&d.x2, x2.data(), nl2) || upload(&d.st, st.data(), nl2) ||
         upload(&d.wq, wq.data(), nl2) || upload(&d.step_ofs, ofs.data(), ofs.size()) ||
         upload(&d.ab, ab.data(), ab.size()) || upload(&d.pm, pm.data(), pm.size()) ||
         upload(&d.roots, roots.data(), roots.size()) || upload(&d.fft_pos, pos.data(), pos.size()) ||
+        upload(&d.any_pos, any_pos.data(), any_pos.size()) ||
         upload(&d.tm, c->tm.data(), c->tm.size()) || (!c->nrm.empty() && upload(&d.nrm, c->nrm.data(), c->nrm.size()))) {
         set_error(2, "device table allocation failed");
         c->gpu_ready = true;
@@ -1313,9 +1317,7 @@ static void scale_output(shtns_cfg c, cplx *Q, long spec_dist, int nf, int inv) 
 // The Legendre kernel runs in chunks of latitude tiles on the compute stream; the FFT of a
 // chunk's latitudes (north and south rows) runs on the second stream as soon as the chunk
 // is done, overlapping the next chunk's Legendre work (matrix cores vs LDS/HBM).
-// V is double (vf == nullptr) or, for the FP32-data entry points, float: vf != nullptr, with
-// vstage an FP64 staging area of nfields * nspat doubles when the register FFT cannot take
-// the length (then the FFT writes vstage and a conversion kernel writes vf).
+// V is double (vf == nullptr) or, for the FP32-data entry points, float (vf).
 // Tables of the sliced (int8) contraction, built on first use by the configuration that owns
 // the device tables (a clone builds them on its source and copies the pointers).
 static bool ensure_i8_tables(shtns_cfg c) {
@@ -1460,12 +1462,12 @@ static size_t synth_scratch_bytes(shtns_cfg c, int nfields) {
 // bytes is used instead of the configuration's scratch; no stream, event or memory is then
 // created (no profiling, no overlapped chunks).
 static void synth_core_on(shtns_cfg c, const cplx *Q, double *V, int ltr, int nfields, long spec_dist, long spat_dist,
-                          double mpos_scale, int lat_weight, int prec, float *vf, double *vstage, void *ext,
+                          double mpos_scale, int lat_weight, int prec, float *vf, void *ext,
                           const SpatPairs *zp);
 // zp: the spatial output goes to interleaved complex fields instead of V (nfields even,
 // synth_pairs_ok(c))
 static void synth_core(shtns_cfg c, const cplx *Q, double *V, int ltr, int nfields, long spec_dist, long spat_dist,
-                       double mpos_scale, int lat_weight, int prec, float *vf = nullptr, double *vstage = nullptr,
+                       double mpos_scale, int lat_weight, int prec, float *vf = nullptr,
                        void *ext = nullptr, const SpatPairs *zp = nullptr) {
     if (nfields <= 0) return;
     if (!c->nrm.empty()) {
@@ -1476,10 +1478,10 @@ static void synth_core(shtns_cfg c, const cplx *Q, double *V, int ltr, int nfiel
         Q = scaled_input(c, Q, spec_dist, nfields, lat_weight /* adjoint of the analysis: 1 / nrm */, 0);
         if (!Q) return;
     }
-    synth_core_on(c, Q, V, ltr, nfields, spec_dist, spat_dist, mpos_scale, lat_weight, prec, vf, vstage, ext, zp);
+    synth_core_on(c, Q, V, ltr, nfields, spec_dist, spat_dist, mpos_scale, lat_weight, prec, vf, ext, zp);
 }
 static void synth_core_on(shtns_cfg c, const cplx *Q, double *V, int ltr, int nfields, long spec_dist, long spat_dist,
-                          double mpos_scale, int lat_weight, int prec, float *vf, double *vstage, void *ext,
+                          double mpos_scale, int lat_weight, int prec, float *vf, void *ext,
                           const SpatPairs *zp) {
     ltr = clamp_ltr(c, ltr);
     const int imlim = imlim_of(c, ltr);
@@ -1535,13 +1537,8 @@ static void synth_core_on(shtns_cfg c, const cplx *Q, double *V, int ltr, int nf
         ProfScope ps(c, PK_FFT_SYNTH, nullptr, false, prof);
         if (!vf) {
             fft_synth_to(c, imlim, nfields, F, four_dist, V, spat_dist, zp, S, c->tune_fft_synth);
-        } else if (!vstage) {
-            launch_fft_synth_wave(&c->d, c->nlat, c->nphi / 2, imlim, nfields, F, four_dist, vf, spat_dist, sp, st, S,
-                                  0, c->nlat);
         } else {
-            launch_fft_synth(&c->d, c->nlat, c->nphi, c->mmax, imlim, nfields, F, four_dist, vstage, c->nspat, sp, st,
-                             S);
-            launch_convert(vstage, c->nspat, vf, spat_dist, c->nspat, nfields, S);
+            launch_fft_synth(&c->d, c->nlat, c->nphi, imlim, nfields, F, four_dist, vf, spat_dist, sp, st, S);
         }
         HIP_OK(hipGetLastError());
         return;
@@ -1570,21 +1567,20 @@ static void synth_core_on(shtns_cfg c, const cplx *Q, double *V, int ltr, int nf
 
 // analysis core: V -> Q.  With 16+ fields the FFTs of 8-field chunks run on the second
 // stream ahead of the Legendre analysis of the previous chunk on the compute stream.
-// V is double (vf == nullptr) or float (vf != nullptr, vstage as in synth_core: when set,
-// vf is first converted into it).
+// V is double (vf == nullptr) or float (vf).
 static void anal_core_on(shtns_cfg c, const double *V, cplx *Q, int ltr, int nfields, long spat_dist, long spec_dist,
-                         double mpos_scale, int lat_weight, int prec, const float *vf, double *vstage,
+                         double mpos_scale, int lat_weight, int prec, const float *vf,
                          const SpatPairs *zp);
 // zp: the spatial input is read from interleaved complex fields instead of V (nfields even)
 static void anal_core(shtns_cfg c, const double *V, cplx *Q, int ltr, int nfields, long spat_dist, long spec_dist,
                       double mpos_scale, int lat_weight, int prec, const float *vf = nullptr,
-                      double *vstage = nullptr, const SpatPairs *zp = nullptr) {
+                      const SpatPairs *zp = nullptr) {
     if (nfields <= 0) return;
-    anal_core_on(c, V, Q, ltr, nfields, spat_dist, spec_dist, mpos_scale, lat_weight, prec, vf, vstage, zp);
+    anal_core_on(c, V, Q, ltr, nfields, spat_dist, spec_dist, mpos_scale, lat_weight, prec, vf, zp);
     scale_output(c, Q, spec_dist, nfields, lat_weight /* analysis: 1 / nrm; adjoint of the synthesis: nrm */);
 }
 static void anal_core_on(shtns_cfg c, const double *V, cplx *Q, int ltr, int nfields, long spat_dist, long spec_dist,
-                         double mpos_scale, int lat_weight, int prec, const float *vf, double *vstage,
+                         double mpos_scale, int lat_weight, int prec, const float *vf,
                          const SpatPairs *zp) {
     ltr = clamp_ltr(c, ltr);
     const int imlim = imlim_of(c, ltr);
@@ -1609,13 +1605,8 @@ static void anal_core_on(shtns_cfg c, const double *V, cplx *Q, int ltr, int nfi
             ProfScope ps(c, PK_FFT_ANAL);
             if (!vf) {
                 fft_anal_from(c, imlim, nfields, 0, V, spat_dist, zp, F, four_dist, S, c->tune_fft_anal);
-            } else if (!vstage) {
-                launch_fft_anal_wave(&c->d, c->nlat, c->nphi / 2, c->mmax, imlim, nfields, vf, spat_dist, F,
-                                     four_dist, sp, st, S, 0, c->nlat);
             } else {
-                launch_convert(vf, spat_dist, vstage, c->nspat, c->nspat, nfields, S);
-                launch_fft_anal(&c->d, c->nlat, c->nphi, c->mmax, imlim, nfields, vstage, c->nspat, F, four_dist, sp,
-                                st, S);
+                launch_fft_anal(&c->d, c->nlat, c->nphi, c->mmax, imlim, nfields, vf, spat_dist, F, four_dist, sp, st, S);
             }
         }
         LegendreArgs a = leg_args(c, ltr, imlim, nfields);
@@ -1759,7 +1750,7 @@ extern "C" void cu_SH_to_spat_batch_noalloc(shtns_cfg c, cplx *Q, double *V, int
         set_error(3, "cu_SH_to_spat_batch_noalloc: no fixed workspace on device %d", c->device);
         return;
     }
-    synth_core(c, Q, V, ltr, nf, spec_dist, spat_dist, 1.0, 0, prec_f64(c), nullptr, nullptr, ws);
+    synth_core(c, Q, V, ltr, nf, spec_dist, spat_dist, 1.0, 0, prec_f64(c), nullptr, ws);
 }
 extern "C" void cu_SH_to_spat(shtns_cfg c, cplx *Q, double *V, int ltr) {
     cu_SH_to_spat_batch(c, Q, V, ltr, 1, c->nlm, c->nspat);
@@ -1772,28 +1763,20 @@ extern "C" void cu_SH_to_spat_float_batch(shtns_cfg c, cplx_f *Q, float *V, int 
     clear_error();
     if (!ready(c, "cu_SH_to_spat_float")) return;
     if (nf <= 0) return;
-    const bool stage = !fft_wave_supported(c->nphi / 2);
-    const size_t qb = (size_t)nf * c->nlm * sizeof(double2);
-    char *base = (char *)xscratch(c, qb + (stage ? (size_t)nf * c->nspat * sizeof(double) : 0));
-    if (!base) return;
-    double2 *qd = (double2 *)base;
+    double2 *qd = (double2 *)xscratch(c, (size_t)nf * c->nlm * sizeof(double2));
+    if (!qd) return;
     launch_convert(reinterpret_cast<const float *>(Q), 2 * spec_dist, reinterpret_cast<double *>(qd), 2L * c->nlm,
                    2L * c->nlm, nf, c->comp_stream);
-    synth_core(c, reinterpret_cast<const cplx *>(qd), nullptr, ltr, nf, c->nlm, spat_dist, 1.0, 0, prec_f32(c), V,
-               stage ? (double *)(base + qb) : nullptr);
+    synth_core(c, reinterpret_cast<const cplx *>(qd), nullptr, ltr, nf, c->nlm, spat_dist, 1.0, 0, prec_f32(c), V);
 }
 extern "C" void cu_spat_to_SH_float_batch(shtns_cfg c, float *V, cplx_f *Q, int ltr, int nf, long spat_dist,
                                           long spec_dist) {
     clear_error();
     if (!ready(c, "cu_spat_to_SH_float")) return;
     if (nf <= 0) return;
-    const bool stage = !fft_wave_supported(c->nphi / 2);
-    const size_t qb = (size_t)nf * c->nlm * sizeof(double2);
-    char *base = (char *)xscratch(c, qb + (stage ? (size_t)nf * c->nspat * sizeof(double) : 0));
-    if (!base) return;
-    double2 *qd = (double2 *)base;
-    anal_core(c, nullptr, reinterpret_cast<cplx *>(qd), ltr, nf, spat_dist, c->nlm, 1.0, 1, prec_f32(c), V,
-              stage ? (double *)(base + qb) : nullptr);
+    double2 *qd = (double2 *)xscratch(c, (size_t)nf * c->nlm * sizeof(double2));
+    if (!qd) return;
+    anal_core(c, nullptr, reinterpret_cast<cplx *>(qd), ltr, nf, spat_dist, c->nlm, 1.0, 1, prec_f32(c), V);
     if (g_last_err) return;
     launch_convert(reinterpret_cast<const double *>(qd), 2L * c->nlm, reinterpret_cast<float *>(Q), 2 * spec_dist,
                    2L * c->nlm, nf, c->comp_stream);
@@ -2031,7 +2014,7 @@ extern "C" void cu_SH_to_spat_cplx_batch(shtns_cfg c, cplx *alm, cplx *z, int nf
     if (direct) {
         const SpatPairs zp{reinterpret_cast<double *>(z), spat_dist};
         synth_core(c, reinterpret_cast<const cplx *>(XY), nullptr, c->lmax, 2 * nf, c->nlm, c->nspat, 1.0, 0,
-                   prec_f64(c), nullptr, nullptr, nullptr, &zp);
+                   prec_f64(c), nullptr, nullptr, &zp);
     } else {
         double *xy = (double *)(base + qb);
         synth_core(c, reinterpret_cast<const cplx *>(XY), xy, c->lmax, 2 * nf, c->nlm, c->nspat, 1.0, 0, prec_f64(c));
@@ -2048,7 +2031,7 @@ extern "C" void cu_spat_cplx_to_SH_batch(shtns_cfg c, cplx *z, cplx *alm, int nf
     if (!XY) return;
     const SpatPairs zp{reinterpret_cast<double *>(z), spat_dist};
     anal_core(c, nullptr, reinterpret_cast<cplx *>(XY), c->lmax, 2 * nf, c->nspat, c->nlm, 1.0, 1, prec_f64(c),
-              nullptr, nullptr, &zp);
+              nullptr, &zp);
     if (g_last_err) return;
     launch_cplx_merge(XY, c->nlm, reinterpret_cast<double2 *>(alm), spec_dist, c->lmax, c->mmax, nf, c->comp_stream);
     HIP_OK(hipGetLastError());

@@ -69,7 +69,9 @@ struct DeviceTables {
     // FFT: roots e^{2 pi i k/nphi}, k < nphi
     double2 *roots = nullptr;
     int *fft_pos = nullptr;    // [M] position of output bin k after the in-place DIF FFT
-    FftPlan plan{};
+    FftPlan plan{};            // radices 4, 2, 3, 5, 7 (LDS-staged kernels specialized on the length)
+    FftPlan any_plan{};        // fewest passes of radices up to 16 (sht_fft_any.hip)
+    int *any_pos = nullptr;    // fft_pos of any_plan
     // vector transforms
 };
 
@@ -238,6 +240,16 @@ bool launch_fft_anal_wave(const DeviceTables *t, int nlat, int M, int mmax, int 
                           long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
                           int lat_end);
 bool fft_wave_supported(int M);
+bool launch_fft_synth_coops_f32(const DeviceTables *t, int nlat, int M, int imlim, int nfields, const double2 *F,
+                                long four_dist, float *V, long spat_dist, long sp, long st, hipStream_t s);
+bool launch_fft_anal_coops_f32(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const float *V,
+                               long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s);
+// single-precision fields (transform in FP64, values converted at load / store), every length
+// and layout
+void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int imlim, int nfields, const double2 *F, long four_dist,
+                      float *V, long spat_dist, long sp, long st, hipStream_t s);
+void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int imlim, int nfields, const float *V,
+                     long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s);
 // block-cooperative register FFT (sht_fft.hip): T = 256/LQ latitudes per block, HBM accesses
 // with the latitude fastest (theta-contiguous layout); M = nphi/2 in {32, 48, ..., 1536}
 bool fft_coop_supported(int M);
@@ -247,7 +259,7 @@ bool launch_fft_synth_coop(const DeviceTables *t, int nlat, int M, int imlim, in
 bool launch_fft_anal_coop(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const double *V,
                           long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
                           int lat_end, int nthreads = 256);
-// any length (t->plan, t->fft_pos), runtime plan in LDS (sht_fft_any.hip); false when the length
+// any length (t->any_plan, t->any_pos), runtime plan in LDS (sht_fft_any.hip); false when the length
 // does not fit a CU's LDS
 bool launch_fft_synth_any(const DeviceTables *t, int nlat, int imlim, int nfields, const double2 *F, long four_dist,
                           double *V, long spat_dist, long sp, long st, hipStream_t s, int lat_base, int lat_end);

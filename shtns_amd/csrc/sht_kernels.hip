@@ -661,33 +661,6 @@ __device__ inline int xcd_group(int bid, int G) {
     return (bid % 8) * (G / 8) + bid / 8;
 }
 
-__device__ void fft_dif_inplace(double2 *buf, int T, int M, const FftPlan &plan, const double2 *__restrict__ roots,
-                                double sgn) {
-    const int N = 2 * M;
-    int Ns = M;
-    for (int s = 0; s < plan.nstages; ++s) {
-        const int p = plan.radix[s];
-        const int q = Ns / p;
-        const int nb = M / p;
-        const int twm = N / Ns;
-        for (int b = threadIdx.x; b < T * nb; b += blockDim.x) {
-            const int t = b % T, bb = b / T;
-            const int g = bb / q, n1 = bb - g * q;
-            double2 *a = buf + (size_t)t * M + (size_t)g * Ns + n1;
-            switch (p) {
-                case 4: dif_butterfly<4>(a, q, n1, twm, roots, N, sgn); break;
-                case 2: dif_butterfly<2>(a, q, n1, twm, roots, N, sgn); break;
-                case 3: dif_butterfly<3>(a, q, n1, twm, roots, N, sgn); break;
-                case 5: dif_butterfly<5>(a, q, n1, twm, roots, N, sgn); break;
-                case 7: dif_butterfly<7>(a, q, n1, twm, roots, N, sgn); break;
-                default: break;
-            }
-        }
-        __syncthreads();
-        Ns = q;
-    }
-}
-
 // Compile-time radix plan (same factor order as the host's factor_fft: 4s, then 2, 3, 5, 7),
 // so kernels specialized on M have all butterfly index arithmetic on constants.
 struct CPlan {
@@ -731,16 +704,14 @@ __device__ inline void fft_dif_stages_c(double2 *buf, const double2 *__restrict_
     }
 }
 
-// MC > 0: length M = MC known at compile time (T latitudes per block, TC); MC == 0: runtime plan.
-template <int MC, int TC>
+// T latitudes of M points per block.
+template <int M, int T>
 __global__ __launch_bounds__(256) void fft_synth_kernel(const double2 *__restrict__ F, long four_dist,
                                                         double *__restrict__ V, long spat_dist,
                                                         const double2 *__restrict__ roots, const int *__restrict__ pos,
-                                                        FftPlan plan, int nlat, int imlim, long sp, long stt, int Trt,
-                                                        int lat_base, int lat_end) {
+                                                        int nlat, int imlim, long sp, long stt, int lat_base,
+                                                        int lat_end) {
     extern __shared__ double2 buf[];
-    const int M = MC ? MC : plan.M;
-    const int T = MC ? TC : Trt;
     const int lat0 = lat_base + xcd_group(blockIdx.x, gridDim.x) * T;
     const int f = blockIdx.y;
     const double2 *Ff = F + (size_t)f * four_dist;
@@ -763,8 +734,7 @@ __global__ __launch_bounds__(256) void fft_synth_kernel(const double2 *__restric
         buf[(size_t)t * M + k] = Z;
     }
     __syncthreads();
-    if constexpr (MC > 0) fft_dif_stages_c<MC, TC, 0>(buf, roots, +1.0);
-    else fft_dif_inplace(buf, T, M, plan, roots, +1.0);
+    fft_dif_stages_c<M, T, 0>(buf, roots, +1.0);
     for (int e = threadIdx.x; e < T * M; e += blockDim.x) {
         const int t = e % T, n = e / T;
         if (t < Tv) {
@@ -776,15 +746,13 @@ __global__ __launch_bounds__(256) void fft_synth_kernel(const double2 *__restric
     }
 }
 
-template <int MC, int TC>
+template <int M, int T>
 __global__ __launch_bounds__(256) void fft_anal_kernel(const double *__restrict__ V, long spat_dist,
                                                        double2 *__restrict__ F, long four_dist,
                                                        const double2 *__restrict__ roots, const int *__restrict__ pos,
-                                                       FftPlan plan, int nlat, int mmax, int imlim, long sp, long stt,
-                                                       int Trt, int lat_base, int lat_end) {
+                                                       int nlat, int mmax, int imlim, long sp, long stt,
+                                                       int lat_base, int lat_end) {
     extern __shared__ double2 buf[];
-    const int M = MC ? MC : plan.M;
-    const int T = MC ? TC : Trt;
     const int lat0 = lat_base + xcd_group(blockIdx.x, gridDim.x) * T;
     const int f = blockIdx.y;
     const double *Vf = V + (size_t)f * spat_dist;
@@ -800,8 +768,7 @@ __global__ __launch_bounds__(256) void fft_anal_kernel(const double *__restrict_
         buf[(size_t)t * M + n] = z;
     }
     __syncthreads();
-    if constexpr (MC > 0) fft_dif_stages_c<MC, TC, 0>(buf, roots, -1.0);
-    else fft_dif_inplace(buf, T, M, plan, roots, -1.0);
+    fft_dif_stages_c<M, T, 0>(buf, roots, -1.0);
     for (int e = threadIdx.x; e < T * (mmax + 1); e += blockDim.x) {
         const int t = e % T, k = e / T;
         if (t >= Tv) continue;
@@ -822,21 +789,10 @@ __global__ __launch_bounds__(256) void fft_anal_kernel(const double *__restrict_
     }
 }
 
-static int fft_lat_per_block(int M) {
-    static const int t_env = getenv("SHTNS_AMD_FFT_T") ? atoi(getenv("SHTNS_AMD_FFT_T")) : 0;
-    int T = (int)(65536 / (16L * M));   // LDS budget of 64 KB per block by default
-    if (t_env > 0) T = t_env;
-    while (T > 1 && 16L * M * T > 160 * 1024) --T;
-    if (T < 1) T = 1;
-    if (T > 8) T = 8;
-    return T;
-}
-
 // latitudes per block of the specialized kernels: 2 while 2 sequences fit in 64 KB of LDS
 static constexpr int fft_tc(int M) { return (32L * M <= 65536) ? 2 : 1; }
 
-#define FFT_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024) X(1536) X(2048) \
-    X(3072) X(4096) X(6144)
+#define FFT_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024) X(1536)
 
 bool lds_fft_specialized(int M) {
 #define LDS_OK(MM) if (M == MM) return true;
@@ -845,14 +801,20 @@ bool lds_fft_specialized(int M) {
     return false;
 }
 
-// FFT kernel for a length, layout and direction: 1 register FFT, one latitude per 2..256
-// lanes (sht_fft.hip); 2 LDS-staged FFT (below); 3 / 4 block-cooperative register FFT with 256
-// / 128 threads, 5 / 6 the same with 8-byte LDS staging and 256 / 512 threads (sht_fft.hip).
+// FFT kernel for a length and layout: 1 register FFT, one latitude per 2..256 lanes
+// (sht_fft.hip); 2 LDS-staged FFT (above); 3 / 4 block-cooperative register FFT with 256 / 128
+// threads, 5 / 6 the same with 8-byte LDS staging and 256 / 512 threads (sht_fft.hip); 7 the
+// runtime-plan FFT of any length (sht_fft_any.hip).
 // The register kernel keeps each latitude's accesses separate, contiguous only in the
-// phi-contiguous layout (sp == 1).  In the theta-contiguous layout, measured at lmax=1023 with
-// 16 fields, kind 5: synthesis 0.29 ms (two blocks per CU; kind 3 0.37, LDS kernel 0.55),
-// analysis 0.33 ms (three blocks per CU; kind 6 0.38, LDS kernel 0.57).
-// kind (autotuner) or SHTNS_AMD_FFT=wave|lds|coop|coop128|coops|coops512 override.
+// phi-contiguous layout (sp == 1).  In the theta-contiguous layout kind 5 is the fastest for
+// M = 256 .. 1536 (lmax=1023, 16 fields: synthesis 0.29 ms, kind 3 0.37, kind 2 0.55; analysis
+// 0.33, kind 6 0.38, kind 2 0.57).  Below, its blocks hold 32 and more latitudes and are too few
+// (lmax=127, one field: 6 blocks): analysis call of 1 / 8 / 48 fields 21.0 / 22.3 / 39.8 us, with
+// kind 7 18.4 / 19.6 / 37.0; synthesis 22.2 / 26.7 / 51.9 us, with kind 7 22.1 / 25.0 / 49.6.
+// Above, a latitude takes more than a wave's lanes: kind 7 (M = 2048, 4 fields: synthesis call
+// 532 us, kind 2 591; M = 3072: 715 us, kind 2 759, kind 1 801).  The choice does not depend on
+// the number of fields: a field's result does not depend on its batch.
+// kind (autotuner) or SHTNS_AMD_FFT=wave|lds|coop|coop128|coops|coops512|any override.
 // threads per block of the cooperative kinds (negative: 8-byte LDS staging)
 static int coop_threads(int kind) { return kind == 4 ? 128 : kind == 5 ? -256 : kind == 6 ? -512 : 256; }
 
@@ -866,14 +828,14 @@ static int fft_choice(int M, long sp, int kind) {
                : !strcmp(env, "coop128")  ? 4
                : !strcmp(env, "coops")    ? 5
                : !strcmp(env, "coops512") ? 6
+               : !strcmp(env, "any")      ? 7
                                           : 0;
+    if (want == 7) return 7;
     if (want == 2 && lds_fft_specialized(M)) return 2;
     if (want >= 3 && want <= 6 && fft_coop_supported(M)) return want;
     if (want == 1 && fft_wave_supported(M)) return 1;
     if (sp == 1 && fft_wave_supported(M)) return 1;
-    if (fft_coop_supported(M)) return 5;
-    if (lds_fft_specialized(M)) return 2;
-    return fft_wave_supported(M) ? 1 : 2;
+    return (sp != 1 && M > 192 && fft_coop_supported(M)) ? 5 : 7;
 }
 
 // hipFuncSetAttribute once per kernel and size: kept out of the launch path so launches can
@@ -901,7 +863,7 @@ void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int mmax, int i
     if (nlat_chunk < 0) { lat_base = 0; nlat_chunk = nlat; }
     const int lat_end = lat_base + nlat_chunk;
     static const bool generic = getenv("SHTNS_AMD_FFT_GENERIC") != nullptr;
-    const int choice = generic ? 2 : fft_choice(M, sp, kind);
+    const int choice = generic ? 7 : fft_choice(M, sp, kind);
     if (choice >= 3 && choice <= 6 &&
         launch_fft_synth_coop(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end,
                               coop_threads(choice)))
@@ -910,16 +872,16 @@ void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int mmax, int i
         launch_fft_synth_wave(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end))
         return;
 #define FFT_SYN_CASE(MM)                                                                                        \
-    if (!generic && M == MM) {                                                                                  \
+    if (M == MM) {                                                                                  \
         constexpr int TC = fft_tc(MM);                                                                          \
         const size_t lds = (size_t)TC * MM * sizeof(double2);                                                   \
         set_lds_limit(fft_synth_kernel<MM, TC>, lds);                                                           \
         hipLaunchKernelGGL((fft_synth_kernel<MM, TC>), dim3((nlat_chunk + TC - 1) / TC, nfields), dim3(256), lds, s, \
-                           F, four_dist, V, spat_dist, t->roots, t->fft_pos, t->plan, nlat, imlim, sp, st, TC,  \
-                           lat_base, lat_end);                                                                  \
+                           F, four_dist, V, spat_dist, t->roots, t->fft_pos, nlat, imlim, sp, st, lat_base,     \
+                           lat_end);                                                                  \
         return;                                                                                                 \
     }
-    FFT_SIZES(FFT_SYN_CASE)
+    if (choice == 2) { FFT_SIZES(FFT_SYN_CASE) }
 #undef FFT_SYN_CASE
     if (!launch_fft_synth_any(t, nlat, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end))
         set_error(2, "no longitude FFT for nphi=%d", nphi);
@@ -954,7 +916,7 @@ void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int im
     if (nlat_chunk < 0) { lat_base = 0; nlat_chunk = nlat; }
     const int lat_end = lat_base + nlat_chunk;
     static const bool generic = getenv("SHTNS_AMD_FFT_GENERIC") != nullptr;
-    const int choice = generic ? 2 : fft_choice(M, sp, kind);
+    const int choice = generic ? 7 : fft_choice(M, sp, kind);
     sp *= es;
     st *= es;
     if (choice >= 3 && choice <= 6 &&
@@ -965,19 +927,41 @@ void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int im
         launch_fft_anal_wave(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base, lat_end))
         return;
 #define FFT_ANA_CASE(MM)                                                                                          \
-    if (!generic && M == MM) {                                                                                    \
+    if (M == MM) {                                                                                    \
         constexpr int TC = fft_tc(MM);                                                                            \
         const size_t lds = (size_t)TC * MM * sizeof(double2);                                                     \
         set_lds_limit(fft_anal_kernel<MM, TC>, lds);                                                              \
         hipLaunchKernelGGL((fft_anal_kernel<MM, TC>), dim3((nlat_chunk + TC - 1) / TC, nfields), dim3(256), lds, s,   \
-                           V, spat_dist, F, four_dist, t->roots, t->fft_pos, t->plan, nlat, mmax, imlim, sp, st, TC, \
-                           lat_base, lat_end);                                                                     \
+                           V, spat_dist, F, four_dist, t->roots, t->fft_pos, nlat, mmax, imlim, sp, st, lat_base, \
+                           lat_end);                                                                     \
         return;                                                                                                   \
     }
-    FFT_SIZES(FFT_ANA_CASE)
+    if (choice == 2) { FFT_SIZES(FFT_ANA_CASE) }
 #undef FFT_ANA_CASE
     if (!launch_fft_anal_any(t, nlat, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base, lat_end))
         set_error(2, "no longitude FFT for nphi=%d", nphi);
+}
+
+// Single-precision fields.  The register kernel where the longitude is contiguous, the
+// cooperative one where the latitude is, the runtime-plan one for other lengths.  (The register
+// kernel's accesses touch a cache line per value in the theta-contiguous layout: 16 fields at
+// lmax=511 85 us, cooperative 50 us.)
+void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int imlim, int nfields, const double2 *F, long four_dist,
+                      float *V, long spat_dist, long sp, long st, hipStream_t s) {
+    const int M = nphi / 2;
+    if (sp == 1 && launch_fft_synth_wave(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat)) return;
+    if (sp != 1 && launch_fft_synth_coops_f32(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s)) return;
+    if (launch_fft_synth_any(t, nlat, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat)) return;
+    set_error(2, "no longitude FFT for nphi=%d", nphi);
+}
+void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int imlim, int nfields, const float *V,
+                     long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s) {
+    const int M = nphi / 2;
+    if (sp == 1 && launch_fft_anal_wave(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat))
+        return;
+    if (sp != 1 && launch_fft_anal_coops_f32(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s)) return;
+    if (launch_fft_anal_any(t, nlat, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat)) return;
+    set_error(2, "no longitude FFT for nphi=%d", nphi);
 }
 
 // ---------------------------------------------------------------------------------------
