@@ -599,7 +599,7 @@ __global__ __launch_bounds__(NTB) void fft_synth_coops(const double2 *__restrict
 // With 256 threads (52 KB of LDS at M = 1536) three blocks fit in a CU's LDS; the register
 // budget of three waves per SIMD (168 VGPRs) lets them all be resident.
 template <int M, int NTB, class TV>
-__global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB == 256 ? 3 : 1))) void fft_anal_coops(const TV *__restrict__ V, long spat_dist,
+__global__ __launch_bounds__(NTB) __attribute__((amdgpu_waves_per_eu(NTB <= 256 ? 3 : 1))) void fft_anal_coops(const TV *__restrict__ V, long spat_dist,
                                                       double2 *__restrict__ F, long four_dist,
                                                       const double2 *__restrict__ roots, int nlat, int mmax,
                                                       int imlim, long sp, long stt, int lat_base, int lat_end,
@@ -861,10 +861,21 @@ static bool coop_offsets_fit(int nlat, int M, int kmax, long sp, long st) {
     return v_bytes < 4294967296.0 && f_bytes < 4294967296.0;
 }
 
+// Blocks of 128 threads (half the latitudes) of the split-exchange kernels where 256-thread ones
+// would leave CUs idle; same arithmetic per latitude, so the same results.
+// One field, calls in us with 256 / 128 threads: lmax=255 synthesis 21.0 / 19.0, analysis 26.5 / 24.2;
+// lmax=511 35.3 / 33.8 and 49.5 / 47.7; lmax=127, nphi=512 19.1 / 19.1.
+static bool coops_few_blocks(int nlat_chunk, int M, int nfields) {
+    const int lq = M / wave_R(M), T = 256 / lq;
+    return (long)((nlat_chunk + T - 1) / T) * nfields < 256;
+}
+
 bool launch_fft_synth_coop(const DeviceTables *t, int nlat, int M, int imlim, int nfields, const double2 *F,
                            long four_dist, double *V, long spat_dist, long sp, long st, hipStream_t s, int lat_base,
                            int lat_end, int nthreads) {
     if (!coop_offsets_fit(nlat, M, imlim, sp, st)) return false;
+    if (nthreads == -256 && coops_few_blocks(lat_end - lat_base, M, nfields))
+        return synth_coops<128, double>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
     if (nthreads == -256)
         return synth_coops<256, double>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end);
     if (nthreads == -512)
@@ -900,6 +911,9 @@ bool launch_fft_anal_coop(const DeviceTables *t, int nlat, int M, int mmax, int 
                           long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s, int lat_base,
                           int lat_end, int nthreads) {
     if (!coop_offsets_fit(nlat, M, std::max(mmax, imlim), sp, st)) return false;
+    if (nthreads == -256 && coops_few_blocks(lat_end - lat_base, M, nfields))
+        return anal_coops<128, double>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
+                                       lat_end);
     if (nthreads == -256)
         return anal_coops<256, double>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, lat_base,
                                lat_end);
@@ -930,12 +944,16 @@ bool launch_fft_anal_wave(const DeviceTables *t, int nlat, int M, int mmax, int 
 // single-precision fields, 256 threads
 bool launch_fft_synth_coops_f32(const DeviceTables *t, int nlat, int M, int imlim, int nfields, const double2 *F,
                                 long four_dist, float *V, long spat_dist, long sp, long st, hipStream_t s) {
-    if (!coop_offsets_fit(nlat, M, imlim, sp, st)) return false;
+    if (!fft_coop_supported(M) || !coop_offsets_fit(nlat, M, imlim, sp, st)) return false;
+    if (coops_few_blocks(nlat, M, nfields))
+        return synth_coops<128, float>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat);
     return synth_coops<256, float>(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat);
 }
 bool launch_fft_anal_coops_f32(const DeviceTables *t, int nlat, int M, int mmax, int imlim, int nfields, const float *V,
                                long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s) {
-    if (!coop_offsets_fit(nlat, M, std::max(mmax, imlim), sp, st)) return false;
+    if (!fft_coop_supported(M) || !coop_offsets_fit(nlat, M, std::max(mmax, imlim), sp, st)) return false;
+    if (coops_few_blocks(nlat, M, nfields))
+        return anal_coops<128, float>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat);
     return anal_coops<256, float>(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat);
 }
 

@@ -942,24 +942,27 @@ void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int im
         set_error(2, "no longitude FFT for nphi=%d", nphi);
 }
 
-// Single-precision fields.  The register kernel where the longitude is contiguous, the
-// cooperative one where the latitude is, the runtime-plan one for other lengths.  (The register
-// kernel's accesses touch a cache line per value in the theta-contiguous layout: 16 fields at
-// lmax=511 85 us, cooperative 50 us.)
+// Single-precision fields.  The register kernel where the longitude is contiguous and for short
+// rows (one field at lmax=63: analysis call 20.1 us, cooperative 22.8), the cooperative one where
+// the latitude is, the runtime-plan one for other lengths.  (The register kernel's accesses touch a
+// cache line per value in the theta-contiguous layout: 8 fields at lmax=511, calls 112 us forward
+// and 111 back, cooperative 89 and 91.)
 void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int imlim, int nfields, const double2 *F, long four_dist,
                       float *V, long spat_dist, long sp, long st, hipStream_t s) {
     const int M = nphi / 2;
-    if (sp == 1 && launch_fft_synth_wave(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat)) return;
-    if (sp != 1 && launch_fft_synth_coops_f32(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s)) return;
+    const bool wave = sp == 1 || M <= 192;
+    if (wave && launch_fft_synth_wave(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat)) return;
+    if (!wave && launch_fft_synth_coops_f32(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s)) return;
     if (launch_fft_synth_any(t, nlat, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, 0, nlat)) return;
     set_error(2, "no longitude FFT for nphi=%d", nphi);
 }
 void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int imlim, int nfields, const float *V,
                      long spat_dist, double2 *F, long four_dist, long sp, long st, hipStream_t s) {
     const int M = nphi / 2;
-    if (sp == 1 && launch_fft_anal_wave(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat))
+    const bool wave = sp == 1 || M <= 192;
+    if (wave && launch_fft_anal_wave(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat))
         return;
-    if (sp != 1 && launch_fft_anal_coops_f32(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s)) return;
+    if (!wave && launch_fft_anal_coops_f32(t, nlat, M, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s)) return;
     if (launch_fft_anal_any(t, nlat, mmax, imlim, nfields, V, spat_dist, F, four_dist, sp, st, s, 0, nlat)) return;
     set_error(2, "no longitude FFT for nphi=%d", nphi);
 }

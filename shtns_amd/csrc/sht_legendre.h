@@ -153,7 +153,7 @@ struct Contract {
 constexpr int kSynthTileBytes = 2 * 4 * 64 * sizeof(double);   // LDS per wave
 // Waves (latitude tiles) per block.  Blocks of four waves whose last ones have no tile leave
 // their SIMDs idle: with six tiles half of the blocks loaded two SIMDs only (matrix cores busy
-// 54%; 32 vector pairs at lmax=511: Legendre synthesis 358 -> 305 us in one-wave blocks), so
+// 54%; 64 fields at lmax=511: synthesis call 672 -> 617 us in one-wave blocks), so
 // other counts than multiples of four take one-wave blocks (lmax=560, 16 fields: call 257 ->
 // 243 us; two-wave ones 257).  One to three fields are bound by latency and keep an order's
 // tiles together (lmax=340, 3 fields: 41.5 us, one-wave blocks 44.3).
@@ -1255,6 +1255,9 @@ inline void anal_launch_few(const LegendreArgs &a, const double2 *F, long four_d
 // other's contraction where their LDS allows ((6,2,4)); at 12 tiles the recurrence buffer
 // leaves one block per CU, and more fields per block amortize those phases.  Six-wave blocks
 // load two of the four SIMDs twice.  With few columns, four waves share an order (latency).
+// Single precision: the recurrence outweighs the contraction, so 12 tiles take one wave each for up
+// to four fields (one field, lmax=1023, longitude-contiguous: analysis call 221 -> 208 us); at 6
+// tiles that gave nothing (one / four fields at lmax=511: 57.7 / 71.4, four waves 57.8 / 71.3).
 // One and two tiles are split by half tiles, which sums in the order of the one- and two-field
 // kernel: there a field's result does not depend on its batch.
 template <int PREC>
@@ -1293,6 +1296,7 @@ void anal_launch_shared(const LegendreArgs &a, const double2 *F, long four_dist,
         } else {
             if (ctn >= 3 && !one) ANAL_SHARED(12, 4, 3, 1);
             else if (ctn >= 2 && !one) ANAL_SHARED(12, 2, 6, 1);
+            else if (PREC > 0) ANAL_SHARED(12, 1, 12, 1);
             else ANAL_SHARED(12, 1, 4, 3);
         }
 #undef ANAL_SHARED
