@@ -1525,14 +1525,14 @@ static void synth_core_on(shtns_cfg c, const cplx *Q, double *V, int ltr, int nf
     const int chunk_tiles = 4;
     const int nchunks = (ntiles + chunk_tiles - 1) / chunk_tiles;
     hipStream_t A = (overlap_enabled() && nchunks > 1 && !vf && !ext && !zp) ? aux_stream(c) : nullptr;
-    {
+    if (A) {
         ProfScope ps(c, PK_LEG_SYNTH, nullptr, false, prof);
         launch_premix(a, reinterpret_cast<const double2 *>(Q), spec_dist, c->lmax, qmix, c->nsteps_total, S);
-    }
-    if (!A) {
+    } else {
         {
             ProfScope ps(c, PK_LEG_SYNTH, nullptr, false, prof);
-            launch_legendre_synth_tiles(a, c->lmax, F, four_dist, qmix, c->nsteps_total, 0, ntiles, S);
+            launch_legendre_synth(a, reinterpret_cast<const double2 *>(Q), spec_dist, c->lmax, F, four_dist, qmix,
+                                  c->nsteps_total, S);
         }
         ProfScope ps(c, PK_FFT_SYNTH, nullptr, false, prof);
         if (!vf) {

@@ -187,6 +187,10 @@ void *noalloc_scratch_ptr(int dev);
 // qmix: scratch of synth_qmix_doubles(nfields, nsteps_total) doubles (pre-mixed coefficients)
 void launch_legendre_synth(const LegendreArgs &a, const double2 *Qlm, long spec_dist, int spec_ltop,
                            double2 *F, long four_dist, double *qmix, int nsteps_total, hipStream_t s);
+// one to three FP64 fields: pre-mix and Legendre synthesis in one kernel; false (nothing
+// launched) for other arguments
+bool launch_legendre_synth_few(const LegendreArgs &a, const double2 *Qlm, long spec_dist, int spec_ltop, double2 *F,
+                               long four_dist, hipStream_t s);
 size_t synth_qmix_doubles(int nfields, int nsteps_total, int want_ncg = 0);
 // analysis block shape (waves, latitude tiles per wave) with a compiled kernel
 bool anal_shape_ok(int nw, int nlr);

@@ -239,6 +239,23 @@ void launch_premix(const LegendreArgs &a, const double2 *Qlm, long spec_dist, in
 #undef PREMIX
 }
 
+// The vector-ALU kernel for one field of any size and for two or three on up to 8 tiles; for two
+// also beyond 12.  Measured (synthesis call, vector / matrix kernel): two fields 9 tiles (lmax=700)
+// 98 / 102 us, 12 tiles (lmax=1023) 158 / 146, 16 tiles (lmax=1365) 315 / 327, 24 tiles (lmax=2047)
+// 1008 / 1070; three fields lmax=340 38 / 46, lmax=511 58 / 62, lmax=700 124 / 113, lmax=1365
+// 520 / 440, lmax=2047 1536 / 1409.  With more fields the step's coefficients, 4 per field, cost
+// the LDS what the matrix kernel's operand tile costs, which all its fields share.
+bool launch_legendre_synth_few(const LegendreArgs &a, const double2 *Q, long spec_dist, int spec_ltop, double2 *F,
+                               long four_dist, hipStream_t s) {
+    if (a.prec != kPrecF64 || a.nfields > 3 || synth_ncg(a.nfields, a.synth_ncg) != 1 || synth_force16()) return false;
+    const int ntl = (a.nlat_2 + 63) / 64;
+    if ((a.nfields == 2 && ntl > 8 && ntl <= 12) || (a.nfields == 3 && ntl > 8)) return false;
+    if (a.nfields == 1) launch_synth_few<1>(a, Q, spec_dist, spec_ltop, F, four_dist, s);
+    else if (a.nfields == 2) launch_synth_few<2>(a, Q, spec_dist, spec_ltop, F, four_dist, s);
+    else launch_synth_few<3>(a, Q, spec_dist, spec_ltop, F, four_dist, s);
+    return true;
+}
+
 void launch_legendre_synth_tiles(const LegendreArgs &a, int spec_ltop, double2 *F, long four_dist, const double *qmix,
                                  int nsteps_total, int tile0, int ntl, hipStream_t s) {
     if (a.prec == kPrecF32) launch_legendre_synth_tiles_f32(a, spec_ltop, F, four_dist, qmix, nsteps_total, tile0, ntl, s);
@@ -578,6 +595,7 @@ void launch_ml_anal(const double *T, const double *w, int nlat, int nl, const do
 
 void launch_legendre_synth(const LegendreArgs &a, const double2 *Qlm, long spec_dist, int spec_ltop,
                            double2 *F, long four_dist, double *qmix, int nsteps_total, hipStream_t s) {
+    if (launch_legendre_synth_few(a, Qlm, spec_dist, spec_ltop, F, four_dist, s)) return;
     launch_premix(a, Qlm, spec_dist, spec_ltop, qmix, nsteps_total, s);
     launch_legendre_synth_tiles(a, spec_ltop, F, four_dist, qmix, nsteps_total, 0, (a.nlat_2 + 63) / 64, s);
 }

@@ -449,6 +449,206 @@ void synth_tiles_launch(const LegendreArgs &a, int spec_ltop, double2 *F, long f
 }
 
 // ---------------------------------------------------------------------------------------
+// Synthesis of one to three fields in FP64, on the vector ALUs.
+//
+// The FP64 matrix and vector instructions share one unit (mixed streams add up to the rate of
+// either), so for few fields the vector form costs the same multiply-adds, 2 (recurrence) +
+// 4 NF (E/O, re/im) per step and latitude pair, without the LDS transposition of every value
+// that the matrix operands need (16 KB per 16 steps x 64 latitudes: at one field the LDS was
+// busier than the unit).  lane = latitude pair, R tiles of 64 per wave, sums in registers; the
+// wave-uniform coefficients of a step (alpha, beta, then E and O of each field) are read from
+// LDS by broadcast, 2 + 4 NF doubles shared by the R tiles.
+// The pre-mix is done here, chunk of CS steps by chunk, by the block's threads (the next
+// chunk's loads in flight during the current one): no separate pass over the coefficients.
+// Same order of summation and same roundings as the matrix-core kernel.
+// One field, synthesis call: lmax=4095 4756 -> 3795 us, lmax=2047 715 -> 545, lmax=511 49 -> 33;
+// three fields at lmax=340 46 -> 38.
+// ---------------------------------------------------------------------------------------
+template <int NF, int R>
+__global__ __launch_bounds__(256) void legendre_synth_few_kernel(
+    const double *__restrict__ xk, const double *__restrict__ x2k, const double *__restrict__ wqk,
+    const int *__restrict__ step_ofs, const double2 *__restrict__ ab, const double4 *__restrict__ pm,
+    const int *__restrict__ i0tab, const double2 *__restrict__ z0tab, const double2 *__restrict__ Q, long spec_dist,
+    int lmax_spec, double2 *__restrict__ F, long four_dist, int mmax, int mres, int nlat, int nlat_2, int ltr, int imlim,
+    int vector_mode, double mpos_scale, int lat_weight, int tile0, int ntl, int nblk) {
+    constexpr int CS = 64, ROW = 2 + 4 * NF;   // steps per chunk, doubles per step
+    __shared__ __attribute__((aligned(16))) double cfs[2][CS][ROW];
+    __shared__ int s_beg[4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nw = blockDim.x >> 6, nt = blockDim.x;
+    const int im = blockIdx.x / nblk, tb = tile0 + (blockIdx.x - im * nblk) * nw * R;   // heavy orders first
+
+    const OrderInfo o = order_info(im, lmax_spec, mmax, mres, (im <= imlim) ? ltr : -1, vector_mode);
+    const int nsteps = (im <= imlim) ? o.nsteps : 0;
+    const int sofs = step_ofs[o.slot], last_row = step_ofs[o.slot + 1] - sofs - 1;
+
+    double x2[R], za[R], zb[R], acc[R][NF][4];
+    double2 sd[R];
+    int i0[R], wmin[R], wlast = 0, wbeg = nsteps;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {   // neighbouring tiles: they start at similar steps
+        const int tile = tb + wave * R + r, k = tile * 64 + lane;
+        const bool kv = tile < tile0 + ntl && k < nlat_2;
+        const int kk = kv ? k : 0;
+        x2[r] = x2k[kk];
+        i0[r] = kv ? min(i0tab[(size_t)o.slot * nlat_2 + kk], nsteps) : nsteps;
+        sd[r] = z0tab[(size_t)o.slot * nlat_2 + kk];
+        za[r] = zb[r] = 0.0;
+        wmin[r] = i0[r];
+        wlast = max(wlast, i0[r] < nsteps ? i0[r] : 0);   // lanes that never start stay zero
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[r][f][c] = 0.0;
+    }
+    auto step = [&](int r, const double *c) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[r][f][e] = fma(zb[r], c[2 + 4 * f + e], acc[r][f][e]);
+        const double zn = fma(fma(c[0], x2[r], c[1]), zb[r], za[r]);
+        za[r] = zb[r];
+        zb[r] = zn;
+    };
+    // mixed coefficients of step ii, field f
+    const double qscale = (im == 0) ? 1.0 : mpos_scale;
+    constexpr int NE = (CS * NF + 63) / 64;   // (step, field) elements per thread of a one-wave block
+    double2 q0[NE], q1[NE], q2[NE], cab[NE];
+    double4 cpm[NE];
+    auto fetch = [&](int ch) {   // loads of chunk ch
+#pragma unroll
+        for (int j = 0; j < NE; ++j) {
+            const int e = threadIdx.x + j * nt;
+            if (j > 0 && j * nt >= CS * NF) break;   // block-uniform
+            const int f = e / CS, ii = ch + e % CS, le = o.mfun + 2 * ii;
+            const bool in = e < CS * NF && ii < nsteps;
+            const double2 *Qf = Q + (size_t)(in ? f : 0) * spec_dist + o.spec_base;
+            const int lc = in ? le : max(o.mfun, 0);
+            const bool any = nsteps > 0;
+            cpm[j] = pm[sofs + min(ii, last_row)];
+            cab[j] = ab[sofs + min(ii, last_row)];
+            q0[j] = (any && in) ? Qf[lc] : make_double2(0.0, 0.0);
+            q1[j] = (any && in && le + 1 <= ltr) ? Qf[lc + 1] : make_double2(0.0, 0.0);
+            q2[j] = (any && in && le + 2 <= ltr) ? Qf[lc + 2] : make_double2(0.0, 0.0);
+        }
+    };
+    auto put = [&](int b) {
+#pragma unroll
+        for (int j = 0; j < NE; ++j) {
+            const int e = threadIdx.x + j * nt;
+            if (j > 0 && j * nt >= CS * NF) break;
+            if (e >= CS * NF) break;
+            const int f = e / CS, s = e % CS;
+            const double4 cf = cpm[j];
+            double4 out;
+            out.x = (cf.x * q0[j].x + cf.y * q2[j].x) * qscale;
+            out.y = (cf.x * q0[j].y + cf.y * q2[j].y) * qscale;
+            out.z = (cf.z * q1[j].x) * qscale;
+            out.w = (cf.z * q1[j].y) * qscale;
+            if (o.real_only) out.y = out.w = 0.0;
+            double *d = &cfs[b][s][2 + 4 * f];
+            d[0] = out.x; d[1] = out.y; d[2] = out.z; d[3] = out.w;
+            if (f == 0) { cfs[b][s][0] = cab[j].x; cfs[b][s][1] = cab[j].y; }
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        for (int off = 32; off >= 1; off >>= 1) {
+            wmin[r] = min(wmin[r], __shfl_xor(wmin[r], off));
+        }
+        wmin[r] = __builtin_amdgcn_readfirstlane(wmin[r]) & ~3;
+        wbeg = min(wbeg, wmin[r]);
+    }
+    for (int off = 32; off >= 1; off >>= 1) wlast = max(wlast, __shfl_xor(wlast, off));
+    wlast = __builtin_amdgcn_readfirstlane(wlast);
+    if (lane == 0) s_beg[wave] = wbeg;
+    __syncthreads();
+    int beg = nsteps;
+    for (int w = 0; w < nw; ++w) beg = min(beg, s_beg[w]);
+    beg = __builtin_amdgcn_readfirstlane(beg) & ~(CS - 1);
+    if (beg < nsteps) {
+        fetch(beg);
+        put(0);
+    }
+    __syncthreads();
+    int b = 0;
+    for (int ch = beg; ch < nsteps; ch += CS, b ^= 1) {
+        const bool more = ch + CS < nsteps;
+        if (more) fetch(ch + CS);
+        const int send = min(CS, nsteps - ch), sbeg = max(0, wbeg - ch);
+        int s4 = sbeg;
+        // some latitude of the wave still starts: tile by tile
+        for (; s4 < send && ch + s4 <= wlast; s4 += 4) {   // rows past nsteps hold zeros
+            const int i = ch + s4;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (i < wmin[r]) continue;   // wave-uniform: not started
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const double *c = cfs[b][s4 + s];
+                    if (i + s == i0[r]) { za[r] = sd[r].x; zb[r] = sd[r].y; }
+                    step(r, c);
+                }
+            }
+        }
+        // all started: the tiles' independent chains side by side, coefficients read once
+        for (; s4 < send; s4 += 2) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                double c[ROW];
+#pragma unroll
+                for (int e = 0; e < ROW; e += 2) {
+                    const double2 v = *reinterpret_cast<const double2 *>(&cfs[b][s4 + s][e]);
+                    c[e] = v.x;
+                    c[e + 1] = v.y;
+                }
+#pragma unroll
+                for (int r = 0; r < R; ++r) step(r, c);
+            }
+        }
+        if (more) put(b ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int tile = tb + wave * R + r, k = tile * 64 + lane;
+        if (tile >= tile0 + ntl || k >= nlat_2) continue;
+        const double x = xk[k];
+        // the middle row of an odd grid is its own mirror: its stored pair weight is halved
+        const double w = lat_weight ? wqk[k] * ((2 * k + 1 == nlat) ? 2.0 : 1.0) : 1.0, wi = (im == 0) ? 0.0 : w;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            double2 *Ff = F + (size_t)f * four_dist + (size_t)im * nlat;
+            const double *a = acc[r][f];
+            Ff[k] = make_double2(fma(x, a[2], a[0]) * w, fma(x, a[3], a[1]) * wi);
+            Ff[nlat - 1 - k] = make_double2(fma(-x, a[2], a[0]) * w, fma(-x, a[3], a[1]) * wi);
+        }
+    }
+}
+
+// Tiles per wave: one up to 12 tiles, then two (the coefficient reads of a step are shared and
+// two chains run side by side): lmax=2047, 1 / 2 fields, call 545 / 976 us, one tile per wave
+// 679 / 1218, three 548 / 991, six 692; lmax=511, one field 33.6, two tiles 35.8.
+template <int NF>
+void launch_synth_few(const LegendreArgs &a, const double2 *Q, long spec_dist, int spec_ltop, double2 *F, long four_dist,
+                      hipStream_t s) {
+    const DeviceTables *t = a.t;
+    const int ntl = (a.nlat_2 + 63) / 64;
+#define SYNTH_FEW(RR)                                                                                              \
+    {                                                                                                              \
+        const int nw = std::min(4, (ntl + RR - 1) / RR), nblk = (ntl + nw * RR - 1) / (nw * RR);                   \
+        hipLaunchKernelGGL((legendre_synth_few_kernel<NF, RR>), dim3((a.mmax + 1) * nblk), dim3(64 * nw), 0, s,    \
+                           t->x, t->x2, t->wq, t->step_ofs, t->ab, t->pm, a.vector_mode ? t->i0v : t->i0,          \
+                           a.vector_mode ? t->z0v : t->z0, Q, spec_dist, spec_ltop, F, four_dist, a.mmax, a.mres,  \
+                           a.nlat, a.nlat_2, a.ltr, a.imlim, a.vector_mode, a.mpos_scale, a.lat_weight, 0, ntl,    \
+                           nblk);                                                                                  \
+    }
+    if (ntl <= 12) SYNTH_FEW(1)
+    else SYNTH_FEW(2)
+#undef SYNTH_FEW
+}
+
+// ---------------------------------------------------------------------------------------
 // Analysis: Q_lm = sum_k w_k P_lm(x_k) F_m(x_k)
 // Block = NW waves for one order im and 4*NCG fields; wave w owns latitude tiles
 // w + NW*r (r < NLR) of 64 pairs, lane = latitude pair.  The weighted E/O values of the
