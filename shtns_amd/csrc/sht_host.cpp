@@ -1258,7 +1258,14 @@ extern "C" int shtns_profile_get(shtns_cfg c, double *ms, int *count) {
 
 // contraction precision for double data / float data (cushtns_set_precision)
 static int prec_f64(shtns_cfg c) { return c->prec >= 0 ? c->prec : kPrecF64; }
-static int prec_f32(shtns_cfg c) { return c->prec >= 0 ? c->prec : kPrecF32; }
+// Float data, no precision chosen: FP64 where the few-field FP64 kernels are faster than the FP32
+// matrix ones, which idle most of their columns: synthesis of one to three fields (lmax=511, one /
+// three fields: 35 / 62 us, FP32 53 / 69; lmax=2047, one: 509, FP32 1095) and analysis of one
+// (lmax=511 51 us, FP32 59; lmax=2047 1117, FP32 1416; two fields 1725, FP32 1667).
+static int prec_f32(shtns_cfg c, int nfields, bool anal) {
+    if (c->prec >= 0) return c->prec;
+    return nfields <= (anal ? 1 : 3) ? kPrecF64 : kPrecF32;
+}
 
 static void *xscratch(shtns_cfg c, size_t bytes) {
     if (bytes <= c->xscratch_bytes) return c->xscratch;
@@ -1767,7 +1774,7 @@ extern "C" void cu_SH_to_spat_float_batch(shtns_cfg c, cplx_f *Q, float *V, int 
     if (!qd) return;
     launch_convert(reinterpret_cast<const float *>(Q), 2 * spec_dist, reinterpret_cast<double *>(qd), 2L * c->nlm,
                    2L * c->nlm, nf, c->comp_stream);
-    synth_core(c, reinterpret_cast<const cplx *>(qd), nullptr, ltr, nf, c->nlm, spat_dist, 1.0, 0, prec_f32(c), V);
+    synth_core(c, reinterpret_cast<const cplx *>(qd), nullptr, ltr, nf, c->nlm, spat_dist, 1.0, 0, prec_f32(c, nf, false), V);
 }
 extern "C" void cu_spat_to_SH_float_batch(shtns_cfg c, float *V, cplx_f *Q, int ltr, int nf, long spat_dist,
                                           long spec_dist) {
@@ -1776,7 +1783,7 @@ extern "C" void cu_spat_to_SH_float_batch(shtns_cfg c, float *V, cplx_f *Q, int 
     if (nf <= 0) return;
     double2 *qd = (double2 *)xscratch(c, (size_t)nf * c->nlm * sizeof(double2));
     if (!qd) return;
-    anal_core(c, nullptr, reinterpret_cast<cplx *>(qd), ltr, nf, spat_dist, c->nlm, 1.0, 1, prec_f32(c), V);
+    anal_core(c, nullptr, reinterpret_cast<cplx *>(qd), ltr, nf, spat_dist, c->nlm, 1.0, 1, prec_f32(c, nf, true), V);
     if (g_last_err) return;
     launch_convert(reinterpret_cast<const double *>(qd), 2L * c->nlm, reinterpret_cast<float *>(Q), 2 * spec_dist,
                    2L * c->nlm, nf, c->comp_stream);
