@@ -1463,12 +1463,12 @@ inline void anal_launch_few(const LegendreArgs &a, const double2 *F, long four_d
 template <int PREC>
 void anal_launch_shared(const LegendreArgs &a, const double2 *F, long four_dist, double2 *Q, long spec_dist,
                         int spec_ltop, hipStream_t s) {
-    const int ntiles = (a.nlat_2 + 63) / 64, ns = (ntiles + 11) / 12, per = (ntiles + ns - 1) / ns;
+    const int ntiles = (a.nlat_2 + 63) / 64;
     const int ctn = (a.nfields + 3) / 4;
     // the tuner's choice: 1 for four fields per block, otherwise as many as the shapes below take
     static const int ncg_env = getenv("SHTNS_AMD_ANAL_NCG") ? atoi(getenv("SHTNS_AMD_ANAL_NCG")) : 0;
     const bool one = (a.anal_ncg ? a.anal_ncg : ncg_env) == 1;
-    if (per > 6 && ctn > 4 && (ctn % 4 == 1 || ctn % 4 == 2) && !one) {
+    if (ntiles > 6 && ctn > 4 && (ctn % 4 == 1 || ctn % 4 == 2) && !one) {
         // shapes of 16 fields: the last one to eight fields in blocks of their own size (in the
         // 16-field blocks their waves would wait for nothing: 24 fields at lmax=850 1462 us)
         const int nf0 = (ctn & ~3) * 4;
@@ -1479,8 +1479,12 @@ void anal_launch_shared(const LegendreArgs &a, const double2 *F, long four_dist,
         anal_launch_shared<PREC>(a1, F + (size_t)nf0 * four_dist, four_dist, Q + (size_t)nf0 * spec_dist, spec_dist, spec_ltop, s);
         return;
     }
-    for (int k = 0; k < ns; ++k) {   // in order on the stream: the later splits add to the first one's result
-#define ANAL_SHARED(...) launch_anal_shared<__VA_ARGS__, PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s, k * per, per, k > 0)
+    // 12 tiles per launch and the rest in one of its own shape (13 tiles as 7 + 7 in 8-tile
+    // blocks: lmax=1067, 4 fields 618 us, as 12 + 1 535; 3 fields 552, 480).  In order on the
+    // stream: the later launches add to the first one's result.
+    for (int tile0 = 0; tile0 < ntiles; tile0 += 12) {
+        const int per = std::min(12, ntiles - tile0);
+#define ANAL_SHARED(...) launch_anal_shared<__VA_ARGS__, PREC>(a, F, four_dist, Q, spec_dist, spec_ltop, s, tile0, per, tile0 > 0)
         if (per <= 1) { if (ctn >= 2 && !one) ANAL_SHARED(1, 2, 2, 1); else ANAL_SHARED(1, 1, 2, 1); }
         else if (per <= 2) ANAL_SHARED(2, 1, 4, 1);
         else if (per <= 3) { if (ctn > 4 && !one) ANAL_SHARED(3, 2, 2, 1); else ANAL_SHARED(3, 1, 4, 1); }
