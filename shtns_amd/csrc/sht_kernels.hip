@@ -826,9 +826,12 @@ bool lds_fft_specialized(int M) {
 // The register kernel keeps each latitude's accesses separate, contiguous only in the
 // phi-contiguous layout (sp == 1).  In the theta-contiguous layout kind 5 is the fastest for
 // M = 256 .. 1536 (lmax=1023, 16 fields: synthesis 0.29 ms, kind 3 0.37, kind 2 0.55; analysis
-// 0.33, kind 6 0.38, kind 2 0.57).  Below, its blocks hold 32 and more latitudes and are too few
-// (lmax=127, one field: 6 blocks): analysis call of 1 / 8 / 48 fields 21.0 / 22.3 / 39.8 us, with
-// kind 7 18.4 / 19.6 / 37.0; synthesis 22.2 / 26.7 / 51.9 us, with kind 7 22.1 / 25.0 / 49.6.
+// 0.33, kind 6 0.38, kind 2 0.57).  Below, its blocks hold 16 and more latitudes, and its analysis
+// loses to kind 7: 192 x 384 grid, call of 1 / 8 / 48 fields 18.1 / 19.3 / 38.4 us, kind 7 16.9 /
+// 17.9 / 35.4.  The synthesis is the faster one down to M = 128: 186 x 384, 1 / 8 / 78 fields
+// 16.6 / 24.3 / 53.4 us, kind 7 17.1 / 28.3 / 60.3; 122 x 256, 16.3 / 19.9 / 36.5, kind 7 17.0 /
+// 21.0 / 38.8; M = 96 (96 x 192) 16.5 / 20.1 / 28.7, kind 7 16.8 / 20.3 / 29.4; M = 72 16.7 / 20.6 /
+// 23.6, kind 7 15.9 / 18.5 / 23.2.
 // Above, a latitude takes more than a wave's lanes: kind 7 (M = 2048, 4 fields: synthesis call
 // 532 us, kind 2 591; M = 3072: 715 us, kind 2 759, kind 1 801).  The choice does not depend on
 // the number of fields: a field's result does not depend on its batch.
@@ -836,7 +839,7 @@ bool lds_fft_specialized(int M) {
 // threads per block of the cooperative kinds (negative: 8-byte LDS staging)
 static int coop_threads(int kind) { return kind == 4 ? 128 : kind == 5 ? -256 : kind == 6 ? -512 : 256; }
 
-static int fft_choice(int M, long sp, int kind) {
+static int fft_choice(int M, long sp, int kind, bool anal) {
     static const char *env = getenv("SHTNS_AMD_FFT");
     int want = kind;
     if (!want && env)
@@ -853,7 +856,7 @@ static int fft_choice(int M, long sp, int kind) {
     if (want >= 3 && want <= 6 && fft_coop_supported(M)) return want;
     if (want == 1 && fft_wave_supported(M)) return 1;
     if (sp == 1 && fft_wave_supported(M)) return 1;
-    return (sp != 1 && M > 192 && fft_coop_supported(M)) ? 5 : 7;
+    return (sp != 1 && M >= (anal ? 256 : 128) && fft_coop_supported(M)) ? 5 : 7;
 }
 
 // hipFuncSetAttribute once per kernel and size: kept out of the launch path so launches can
@@ -881,7 +884,7 @@ void launch_fft_synth(const DeviceTables *t, int nlat, int nphi, int mmax, int i
     if (nlat_chunk < 0) { lat_base = 0; nlat_chunk = nlat; }
     const int lat_end = lat_base + nlat_chunk;
     static const bool generic = getenv("SHTNS_AMD_FFT_GENERIC") != nullptr;
-    const int choice = generic ? 7 : fft_choice(M, sp, kind);
+    const int choice = generic ? 7 : fft_choice(M, sp, kind, false);
     if (choice >= 3 && choice <= 6 &&
         launch_fft_synth_coop(t, nlat, M, imlim, nfields, F, four_dist, V, spat_dist, sp, st, s, lat_base, lat_end,
                               coop_threads(choice)))
@@ -910,7 +913,7 @@ bool launch_fft_synth_pairs(const DeviceTables *t, int nlat, int nphi, int imlim
                             long fpart, double *V, long spat_dist, long sp, long st, hipStream_t s, int kind, bool dry) {
     const int M = nphi / 2;
     if (getenv("SHTNS_AMD_FFT_GENERIC") || !fft_coop_supported(M)) return false;
-    const int choice = fft_choice(M, sp, kind);
+    const int choice = fft_choice(M, sp, kind, false);
     if (choice != 5 && choice != 6) return false;
     return launch_fft_synth_coops_pairs(t, nlat, M, imlim, nf, F, fdist, fpart, V, spat_dist, 2 * sp, 2 * st, s,
                                         coop_threads(choice), dry);
@@ -921,7 +924,7 @@ bool launch_fft_anal_pairs(const DeviceTables *t, int nlat, int nphi, int mmax, 
                            bool dry) {
     const int M = nphi / 2;
     if (getenv("SHTNS_AMD_FFT_GENERIC") || !fft_coop_supported(M)) return false;
-    const int choice = fft_choice(M, sp, kind);
+    const int choice = fft_choice(M, sp, kind, true);
     if (choice != 5 && choice != 6) return false;
     return launch_fft_anal_coops_pairs(t, nlat, M, mmax, imlim, nf, V, spat_dist, F, fdist, fpart, 2 * sp, 2 * st, s,
                                        coop_threads(choice), dry);
@@ -934,7 +937,7 @@ void launch_fft_anal(const DeviceTables *t, int nlat, int nphi, int mmax, int im
     if (nlat_chunk < 0) { lat_base = 0; nlat_chunk = nlat; }
     const int lat_end = lat_base + nlat_chunk;
     static const bool generic = getenv("SHTNS_AMD_FFT_GENERIC") != nullptr;
-    const int choice = generic ? 7 : fft_choice(M, sp, kind);
+    const int choice = generic ? 7 : fft_choice(M, sp, kind, true);
     sp *= es;
     st *= es;
     if (choice >= 3 && choice <= 6 &&
