@@ -638,7 +638,8 @@ class sht:
 
     def set_precision(self, prec):
         """Precision of the Legendre contraction on the GPU: SHT_PREC_F64, SHT_PREC_F32,
-        SHT_PREC_SPLIT or SHT_PREC_AUTO (FP64 for double data, FP32 for float data)."""
+        SHT_PREC_SPLIT or SHT_PREC_AUTO (FP64 for double data; for float data FP32, or FP64
+        where that is faster: few fields)."""
         if _lib.load().cushtns_set_precision(self._cfg, int(prec)) != 0:
             _lib.check_error("set_precision")
 

@@ -4,7 +4,7 @@
 //
 // A block holds T latitudes (a power of two) of M complex points.  Bound: LDS traffic and the
 // latency of its phases, so the plan takes few passes of large radices (up to 16) done in
-// registers: M = 360 is 12 x 15 x 2 -> two exchanges less than radices 4, 2, 3, 3, 5; twiddles
+// registers: three for M = 360, where radices up to 5 take five; twiddles
 // are powers of few table values (twiddles<P>); the index arithmetic of a butterfly is one
 // multiplication by a reciprocal; global loads are issued in batches of four, with the
 // latitude fastest on the Fourier side, and the latitude or the longitude fastest on the

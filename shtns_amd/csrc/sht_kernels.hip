@@ -14,8 +14,9 @@
 //   Each lane starts its recurrence at a precomputed step i0 with precomputed values
 //   (seed tables), so no extended-exponent arithmetic is needed in the hot loop.
 //
-// FFT step (per latitude): real FFT of length nphi as a complex FFT of length nphi/2 in LDS,
-//   in-place mixed-radix (2,3,4,5) decimation in frequency; theta-contiguous global layout.
+// FFT step (per latitude): real FFT of length nphi as a complex FFT of length nphi/2.  The
+//   LDS-staged kernels of compiled lengths are here, the register, cooperative and runtime-plan
+//   ones in sht_fft.hip and sht_fft_any.hip; fft_choice picks.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
